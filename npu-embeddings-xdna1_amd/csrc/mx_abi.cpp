@@ -248,7 +248,7 @@ int take_data_error(mx_stream *s, int *flags) {
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
   if (e != hipSuccess) return hip_fail(e, "reading the refusal flag");
   *flags = h[0];
-  if (h[1] > 0) s->last_rows = h[1];
+  s->saw_rows(h[1], s->plan_bound);
   if (h[0]) {
     e = hipMemsetAsync(s->err_dev, 0, sizeof(int), s->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);

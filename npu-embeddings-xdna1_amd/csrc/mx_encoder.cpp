@@ -1350,6 +1350,7 @@ int pass_plan(mx_encoder *enc, Pass &p) {
   if (e == hipSuccess)
     e = mxk::pack_plan(p.w.kv_len, p.B, p.w.seq_start, p.w.seq_start + p.B + 1, p.s->stream,
                        p.s->err_dev + 1);
+  if (e == hipSuccess) p.s->plan_bound = p.B * p.S;
   return e == hipSuccess ? MX_OK : hip_fail(e, "embed launch");
 }
 
@@ -1389,9 +1390,9 @@ int pass_rows(mx_encoder *enc, Pass &p, Carver *carve) {
                          p.s->stream);
       if (e == hipSuccess) e = hipStreamSynchronize(p.s->stream);
       total = t;
-      if (e == hipSuccess && t > 0) p.s->last_rows = t;
+      if (e == hipSuccess) p.s->saw_rows(t, B * S);
     } else {
-      enc->live = mx::Live{p.w.seq_start + B, p.s->last_rows};
+      enc->live = mx::Live{p.w.seq_start + B, p.s->expected_rows(B * S)};
       enc->live_bound = B * S;
     }
     if (e != hipSuccess) return hip_fail(e, "reading the packed row count");
