@@ -176,6 +176,8 @@ hipError_t gemm_lds_launch(const GemmArgs &a, int grid, hipStream_t s);
 hipError_t gemm_lds_deep_launch(const GemmArgs &a, int grid, hipStream_t s);
 hipError_t gemm_lds_128_deep_launch(const GemmArgs &a, int grid, hipStream_t s);
 hipError_t gemm_lds_nc_launch(const GemmArgs &a, int grid, hipStream_t s);
+template <int BM, int BN, int WGM, int WGN, int NS, int RB>
+hipError_t gemm_lds16_launch(const GemmArgs &a, int grid, hipStream_t s);
 
 namespace {
 
@@ -186,7 +188,11 @@ enum GemmPath {
   PATH_LDS_128x256,
   PATH_LDS_128x128,
   PATH_LDS_256x256_DEEP,
-  PATH_LDS_128x128_DEEP
+  PATH_LDS_128x128_DEEP,
+  PATH_LDS16_128x128,      // 8 waves, 128-byte slabs, one block per CU
+  PATH_LDS16_64x64,        // 256-byte slabs, three slots, one block per CU
+  PATH_LDS16_64x64_PAIR,   // 256-byte slabs, two slots, two blocks per CU
+  PATH_LDS16_64x64_RB128   // 128-byte slabs, four slots, two blocks per CU
 };
 
 // The 256 x 256 tile on 128-byte slabs: a bf16 C without a residual or an
@@ -203,22 +209,93 @@ bool lds_path_ok(const GemmArgs &a) {
          (!a.residual || (uintptr_t)a.residual % 16 == 0);
 }
 
+// The least estimated time over the paths whose C is staged compactly
+// (deep_ok). A launch of T tiles runs n = ceil(T / CUs) of them on the fullest
+// CU, one after another or (two blocks per CU) in pairs, so
+//   us = start + K * (pair * (n / 2) + one * (n % 2)) + n * tile
+//        (+ n * res: an fp32 C with a residual),
+// `one` and `pair` the cost per K of one tile on a CU and of two. Fitted to 220
+// products on an MI355X (M 100 to 9000, K and N 384 to 5120, weights rotating
+// over eight copies; 8-9 % rms per path). Against the tile areas alone, by which these
+// products took a tile before, the choice takes 0.73 of the time in the
+// geometric mean over them: 700 x 1024 x 4096 40.7 -> 16.3 us (K = 4096),
+// 1500 x 768 x 768 11.1 -> 7.9, 3000 x 1280 x 5120 with a residual 55 -> 51.
+// The worst product loses 4 % (6000 x 384 x 384, 7.2 -> 7.5 us). The bounds on
+// K keep a tile at least as deep as the ring: a ring that held slabs of three
+// tiles would hold two tiles' epilogue vectors in one place. 64-column tiles
+// take whole column tiles only (every layer of a model has them).
+GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
+  struct Cost {
+    GemmPath path;
+    int bm, bn;
+    double start, one, pair, tile, res;
+  };
+  static const Cost costs[] = {
+      {PATH_LDS_256x256_DEEP, 256, 256, 3.27, .0198, .0396, 3.28, 3.84},
+      {PATH_LDS_256x192, 256, 192, 1.73, .0183, .0366, 4.54, 2.54},
+      {PATH_LDS_128x256, 128, 256, 0.00, .0150, .0300, 5.11, 1.73},
+      {PATH_LDS_128x128_DEEP, 128, 128, 0.63, .0103, .0135, 2.55, 2.64},
+      {PATH_LDS16_128x128, 128, 128, 1.22, .0082, .0164, 2.94, 1.44},
+      {PATH_LDS16_64x64_PAIR, 64, 64, 1.64, .0052, .0061, 0.86, 0.36},
+      {PATH_LDS16_64x64, 64, 64, 2.16, .0036, .0072, 0.77, 1.14},
+      {PATH_LDS16_64x64_RB128, 64, 64, 1.85, .0056, .0070, 0.80, 0.70}};
+  const int64_t cus = cu_count();
+  GemmPath best = PATH_LDS_256x256_DEEP;
+  double best_t = 0.0;
+  for (const Cost &c : costs) {
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    switch (c.path) {
+      case PATH_LDS_256x192:  // 96-column waves cannot pair the gated FFN's blocks
+        if (glu) continue;
+        break;
+      case PATH_LDS_128x128_DEEP:
+        // Below K = 512 the pairs' gain on the 128 x 256 tile is 1 us in 12.
+        if (K < 512 && !glu) continue;
+        break;
+      case PATH_LDS16_128x128:
+        if (glu || K < 256) continue;
+        break;
+      case PATH_LDS16_64x64:
+        if (K % 128 || K < 384 || glu || N % 64) continue;
+        break;
+      case PATH_LDS16_64x64_PAIR:
+        if (K % 128 || K < 256 || glu || N % 64) continue;
+        break;
+      case PATH_LDS16_64x64_RB128:
+        // Only where K has no 256-byte slabs: they halve the barriers per K.
+        if (K % 128 == 0 || K < 256 || glu || N % 64) continue;
+        break;
+      default: break;
+    }
+    const int64_t n = (tiles + cus - 1) / cus;
+    const double t = c.start + (double)K * (c.pair * (double)(n / 2) + c.one * (double)(n % 2)) +
+                     (double)n * (c.tile + (res ? c.res : 0.0));
+    if (best_t == 0.0 || t < best_t) {
+      best = c.path;
+      best_t = t;
+    }
+  }
+  // A few tiles of the gated FFN: the 64-byte form keeps three slabs in flight
+  // ahead, not one, and a launch this small waits on every slab's load.
+  if (best == PATH_LDS_128x128_DEEP && glu && ((M + 127) / 128) * ((N + 127) / 128) * 8 <= cus)
+    return PATH_LDS_128x128;
+  return best;
+}
+
 GemmPath pick(const GemmArgs &a) {
   if (!lds_path_ok(a)) return PATH_STAGED;
   static const GemmPath paths[] = {PATH_LDS_256x256, PATH_LDS_256x192, PATH_LDS_128x256,
                                    PATH_LDS_128x128};
-  const bool deep = deep_ok(a);
   const int64_t m = gemm_pick_rows(a.M, a.m_hint);
-  int t = gemm_lds_tile(m, a.N, deep);
-  if (t == 1 && a.epilogue >= EPI_GLU_SILU) t = 0;  // 96-column waves cannot pair blocks
-  if (t == 0 && deep) return PATH_LDS_256x256_DEEP;
-  // The 128 x 128 tile on 128-byte slabs keeps one slab in flight ahead, the
-  // 64-byte form three: a launch of a few tiles per XCD (the CLS-pruned last
-  // layer's 64-row GEMMs) waits on every slab's load and runs faster with
-  // three ahead. Both run the same MFMA chain over K for every element.
-  if (t == 3 && deep && a.c_bf16 && !a.residual &&
-      ((m + 127) / 128) * ((a.N + 127) / 128) * 8 > cu_count())
-    return PATH_LDS_128x128_DEEP;
+  const bool glu = a.epilogue >= EPI_GLU_SILU;
+  if (deep_ok(a)) return pick_deep(m, a.N, a.K, a.residual != nullptr, glu);
+  // An fp32 C of few tiles (the ViT's patches): one small tile per CU.
+  if (!a.c_bf16 && !a.residual && a.epilogue == 0 && a.K % 128 == 0 && a.K >= 384 &&
+      a.N % 64 == 0 &&
+      ((a.M + 63) / 64) * (a.N / 64) <= cu_count())
+    return PATH_LDS16_64x64;
+  int t = gemm_lds_tile(m, a.N, false);
+  if (t == 1 && glu) t = 0;  // 96-column waves cannot pair blocks
   return paths[t];
 }
 
@@ -308,6 +385,10 @@ const char *gemm_plan_name(int64_t M, int64_t N, int64_t K, bool c_bf16, bool re
     case PATH_LDS_256x192: return "lds_256x192x32_w64x96_ns4_persistent";
     case PATH_LDS_128x256: return "lds_128x256x32_w64x64_ns4_persistent";
     case PATH_LDS_128x128: return "lds_128x128x32_w64x64_ns4_persistent";
+    case PATH_LDS16_128x128: return "lds_128x128x64_w64x32_ns4_mfma16_persistent";
+    case PATH_LDS16_64x64: return "lds_64x64x128_w32x32_ns3_mfma16_persistent";
+    case PATH_LDS16_64x64_PAIR: return "lds_64x64x128_w32x32_ns2_mfma16_persistent";
+    case PATH_LDS16_64x64_RB128: return "lds_64x64x64_w32x32_ns4_mfma16_persistent";
     default: return "staged_128x128x64_w64x64";
   }
 }
@@ -326,7 +407,13 @@ hipError_t gemm(const GemmArgs &a, hipStream_t s) {
   if (a.epilogue >= EPI_GLU_SILU && (p == PATH_STAGED || a.N % 64)) return hipErrorInvalidValue;
   switch (p) {
     case PATH_LDS_256x256_DEEP: return gemm_lds_deep_launch(a, cu_count(), s);
-    case PATH_LDS_128x128_DEEP: return gemm_lds_128_deep_launch(a, cu_count(), s);
+    case PATH_LDS_128x128_DEEP: return gemm_lds_128_deep_launch(a, 2 * cu_count(), s);
+    case PATH_LDS16_128x128: return gemm_lds16_launch<128, 128, 2, 4, 4, 128>(a, cu_count(), s);
+    case PATH_LDS16_64x64: return gemm_lds16_launch<64, 64, 2, 2, 3, 256>(a, cu_count(), s);
+    case PATH_LDS16_64x64_PAIR:
+      return gemm_lds16_launch<64, 64, 2, 2, 2, 256>(a, 2 * cu_count(), s);
+    case PATH_LDS16_64x64_RB128:
+      return gemm_lds16_launch<64, 64, 2, 2, 4, 128>(a, 2 * cu_count(), s);
     case PATH_LDS_256x256: return gemm_lds_launch<256, 256, 2, 4, 3>(a, cu_count(), s);
     case PATH_LDS_256x192: return gemm_lds_launch<256, 192, 4, 2, 4>(a, cu_count(), s);
     case PATH_LDS_128x256: return gemm_lds_launch<128, 256, 2, 4, 4>(a, cu_count(), s);

@@ -20,14 +20,28 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_lds_k(
       rows_dev);
 }
 
+// The body's 16 x 16 MFMA form.
+template <int BM, int BN, int WGM, int WGN, int NS, int EPI, bool RES, bool CBF, int RB>
+__global__ __launch_bounds__(WGM *WGN * 64, 2) void gemm_lds16_k(
+    const uint16_t *__restrict__ A, int64_t lda, const uint16_t *__restrict__ Wt, int M, int N,
+    int K, const float *__restrict__ bias, const float *residual, void *C, int64_t ldc,
+    int tiles_m, int tiles_n, const int32_t *rows_dev) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  gemm_lds_body<BM, BN, WGM, WGN, NS, EPI, RES, CBF, false, false, RB, true>(
+      A, lda, Wt, M, N, K, bias, residual, C, ldc, tiles_m, tiles_n, nullptr, nullptr, smem,
+      rows_dev);
+}
+
 }  // namespace
 
 namespace mxk {
 
-template <int BM, int BN, int WGM, int WGN, int NS, int EPI, bool RES, bool CBF, int RB = 64>
+template <int BM, int BN, int WGM, int WGN, int NS, int EPI, bool RES, bool CBF, int RB = 64,
+          bool M16 = false>
 hipError_t gemm_lds_launch_t(const GemmArgs &a, int grid, hipStream_t s) {
   using Cfg = LdsCfg<BM, BN, WGM, WGN, NS, false, stg_kind(CBF, RES), RB>;
   auto kern = gemm_lds_k<BM, BN, WGM, WGN, NS, EPI, RES, CBF, RB>;
+  if constexpr (M16) kern = gemm_lds16_k<BM, BN, WGM, WGN, NS, EPI, RES, CBF, RB>;
   static bool attr_set = false;
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(
@@ -104,8 +118,19 @@ hipError_t gemm_lds_deep_launch(const GemmArgs &a, int grid, hipStream_t s) {
 
 // The 128 x 128 tile on 128-byte slabs (two 32 KB slots: the LDS of the
 // 64-byte form's four, half the barriers per K) for a bf16 C without a
-// residual.
+// residual or an fp32 C with one. 74-75 KB of LDS: two blocks share a CU, so
+// `grid` may be twice the CUs; the second block's MFMAs run under the first
+// one's barriers and epilogue (3940 x 1280 x 5120, fp32 C with a residual:
+// 94.8 us on the 64-byte form, 74.7 so; 6000 x 1280 x 5120, bf16 C: 110 -> 79).
 hipError_t gemm_lds_128_deep_launch(const GemmArgs &a, int grid, hipStream_t s) {
+  if (!a.c_bf16 && a.residual) {
+    switch (a.epilogue) {
+      case 0: return gemm_lds_launch_t<128, 128, 2, 2, 2, 0, true, false, 128>(a, grid, s);
+      case 1: return gemm_lds_launch_t<128, 128, 2, 2, 2, 1, true, false, 128>(a, grid, s);
+      case 2: return gemm_lds_launch_t<128, 128, 2, 2, 2, 2, true, false, 128>(a, grid, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   if (!a.c_bf16 || a.residual) return hipErrorInvalidValue;
   switch (a.epilogue) {
     case 0: return gemm_lds_launch_t<128, 128, 2, 2, 2, 0, false, true, 128>(a, grid, s);
@@ -117,6 +142,29 @@ hipError_t gemm_lds_128_deep_launch(const GemmArgs &a, int grid, hipStream_t s) 
       return gemm_lds_launch_t<128, 128, 2, 2, 2, EPI_GLU_GELU, false, true, 128>(a, grid, s);
     default: return hipErrorInvalidValue;
   }
+}
+
+// The 16 x 16 MFMA forms (gemm_path() says which product takes which), one
+// tile configuration, an activation and an optional fp32 residual.
+template <int BM, int BN, int WGM, int WGN, int NS, int RB>
+hipError_t gemm_lds16_launch(const GemmArgs &a, int grid, hipStream_t s) {
+#define MX_LDS16_EPI(E)                                                                      \
+  if (a.epilogue == E) {                                                                     \
+    if (a.c_bf16 && !a.residual)                                                             \
+      return gemm_lds_launch_t<BM, BN, WGM, WGN, NS, E, false, true, RB, true>(a, grid, s);   \
+    if (!a.c_bf16 && a.residual)                                                             \
+      return gemm_lds_launch_t<BM, BN, WGM, WGN, NS, E, true, false, RB, true>(a, grid, s);   \
+  }
+  MX_LDS16_EPI(0)
+  MX_LDS16_EPI(1)
+  MX_LDS16_EPI(2)
+#undef MX_LDS16_EPI
+  // An fp32 C without a residual (4.5 KB of staging a wave) on one form alone.
+  if constexpr (BM == 64 && NS == 3) {
+    if (a.epilogue == 0 && !a.c_bf16)
+      return gemm_lds_launch_t<BM, BN, WGM, WGN, NS, 0, false, false, RB, true>(a, grid, s);
+  }
+  return hipErrorInvalidValue;
 }
 
 // A narrowed C (EPI_NARROW_C; no residual): the 256 x 256 tile on 64-byte
@@ -151,5 +199,9 @@ template hipError_t gemm_lds_launch<256, 256, 2, 4, 3>(const GemmArgs &, int, hi
 template hipError_t gemm_lds_launch<128, 256, 2, 4, 4>(const GemmArgs &, int, hipStream_t);
 template hipError_t gemm_lds_launch<128, 128, 2, 2, 4>(const GemmArgs &, int, hipStream_t);
 template hipError_t gemm_lds_launch<256, 192, 4, 2, 4>(const GemmArgs &, int, hipStream_t);
+template hipError_t gemm_lds16_launch<128, 128, 2, 4, 4, 128>(const GemmArgs &, int, hipStream_t);
+template hipError_t gemm_lds16_launch<64, 64, 2, 2, 2, 256>(const GemmArgs &, int, hipStream_t);
+template hipError_t gemm_lds16_launch<64, 64, 2, 2, 3, 256>(const GemmArgs &, int, hipStream_t);
+template hipError_t gemm_lds16_launch<64, 64, 2, 2, 4, 128>(const GemmArgs &, int, hipStream_t);
 
 }  // namespace mxk

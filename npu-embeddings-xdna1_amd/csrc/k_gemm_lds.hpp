@@ -27,7 +27,7 @@
 // same rounding before anything else.
 //
 // Grid. One block per CU walks a list of BM x BN output tiles; its slabs
-// (RB = 64 or 128 bytes of K per row: 32 or 64 bf16, 64 or 128 int8; 128-byte
+// (RB = 64, 128 or 256 bytes of K per row: 32 or 64 bf16, 64 or 128 int8; 128-byte
 // rows make every load request a whole 128-byte line and halve the barriers
 // per K, and need two 64 KB slots for a 256 x 256 tile) form one sequence across tile
 // boundaries, so the ring keeps loading the next tile's first slabs while the
@@ -84,12 +84,29 @@
 // residual load) of a wave covers whole 128-byte (fp32) or 64-byte (bf16) row
 // segments instead of 16-byte pieces of 32 rows.
 //
+// 16 x 16 MFMAs (M16). A wave tile of one or two 32 x 32 blocks has too few
+// MFMAs per k-step to cover its own LDS reads, loads and barriers: a lone wave
+// of 32 x 32 spent ~650 cycles on a 64-deep slab, whatever its loads, reads or
+// MFMAs were reduced to -- the issue of one wave's ~100 instructions, most of
+// them fixed per slab. The form for such tiles therefore (a) takes slabs of up
+// to 256 bytes per row, which halves the fixed part per K, (b) reads slab s +
+// 1 into one whole-slab register set while slab s's MFMAs run from the other,
+// and issues slab s + NS between them, and (c) uses v_mfma_f32_16x16x32_bf16
+// (v_mfma_i32_16x16x64_i8), four independent chains per 32 x 32 block with 30
+// cycles from one product to the next where the 32 x 32 form has one chain of
+// 49. The 16 x 16 form of 32 K adds the same products in the same order as two
+// 32 x 32 ones of 16 K: C's bits do not depend on the form. A 64 x 64 tile of
+// four such waves takes 0.15 us per 64 K against 0.63 for the 128 x 128 tile
+// that served small products before (100 x 4096 x 1024: 40.6 -> 15.5 us).
+//
 // Requirements (the launchers check them; bf16 shapes outside them go to
 // k_gemm.hip's kernel): K a multiple of the slab depth and at least NS slabs,
 // N % 4 == 0, a bias (bf16; optional for int8), 16-byte aligned operands.
 // Rows past M (or N) are fetched from a clamped, in-bounds row and never
 // stored.
 #pragma once
+
+#include <type_traits>
 
 #include "mx_common.hpp"
 #include "mx_kernels.hpp"
@@ -110,7 +127,7 @@ constexpr int STG_ROWB = 144;  // staging row: 32 fp32 + 16 bytes of padding
 // The epilogue's staging per wave (stg_kind): 1 packed bf16 32-row blocks (a
 // bf16 C without a residual), 2 KB; 2 fp32 16-row half blocks (an fp32 C with
 // a residual), 2.25 KB; 0 fp32 32-row blocks (the rest), 4.5 KB. RB: bytes of
-// K per slab row, 64 or 128.
+// K per slab row, 64, 128 or 256.
 constexpr int stg_kind(bool cbf, bool res) { return cbf && !res ? 1 : (res && !cbf ? 2 : 0); }
 
 template <int BM, int BN, int WGM, int WGN, int NS, bool I8, int STG, int RB = 64>
@@ -145,18 +162,18 @@ struct LdsCfg {
   static_assert(BIAS_PER_WAVE % 4 == 0 && BIAS_PER_WAVE <= 256, "bias piece: 16-byte lanes");
   static_assert(ROWS_PER_WAVE <= 64, "a_scale piece: one row per lane");
   static_assert(LDS <= 160 * 1024, "gfx950 LDS is 160 KB");
-  static_assert(RB == 64 || RB == 128, "slab rows of 64 or 128 bytes");
+  static_assert(RB == 64 || RB == 128 || RB == 256, "slab rows of 64, 128 or 256 bytes");
   static_assert(NS >= 2 && LOADS_HI * (NS - 2) < 64, "vmcnt holds at most 63");
 };
 
 // Position of logical 16-byte chunk c in slab row r (an involution in c).
 // Sixteen lanes of a ds_read_b128 phase read rows r..r+15 at one logical
 // chunk; a row of RB bytes spans RB/4 banks, so row r starts at bank
-// 16 * (r % 4) (RB = 64) or 32 * (r % 2) (RB = 128), and the XOR spreads the
-// sixteen reads over all 64 banks.
+// 16 * (r % 4) (RB = 64), 32 * (r % 2) (RB = 128) or 0 (RB = 256), and the XOR
+// spreads the sixteen reads over all 64 banks.
 template <int RB>
 __device__ __forceinline__ int chunk_pos(int c, int r) {
-  return RB == 64 ? c ^ ((r >> 2) & 3) : c ^ ((r >> 1) & 7);
+  return RB == 64 ? c ^ ((r >> 2) & 3) : RB == 128 ? c ^ ((r >> 1) & 7) : c ^ (r & 15);
 }
 
 // s_waitcnt vmcnt(N), other counters untouched.
@@ -195,25 +212,19 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 
 // Wait until this wave's loads of the next slab have landed: at most the
 // loads of the `later` slabs issued after it (LOADS each) may stay in flight,
-// plus `extra` younger operations (the stores of an epilogue issued after that
-// slab's loads). vmcnt counts loads and stores in issue order.
-template <int LOADS, int NS, int EXTRA>
+// plus EXTRA younger operations (the stores of an epilogue issued after that
+// slab's loads). vmcnt counts loads and stores in issue order. `ahead`: the
+// slabs issued after the next one; all but the last NS - 2 slabs of a block
+// have NS - 2 of them.
+template <int LOADS, int LATER, int EXTRA>
 __device__ __forceinline__ void wait_slab(int ahead, bool extra) {
-  if (ahead >= NS - 2) {
+  if (ahead >= LATER || LATER == 0) {
     if (extra)
-      wait_vmcnt<LOADS *(NS - 2) + EXTRA>();
+      wait_vmcnt<LOADS * LATER + EXTRA>();
     else
-      wait_vmcnt<LOADS *(NS - 2)>();
-  } else if (NS > 3 && ahead == NS - 3) {
-    if (extra)
-      wait_vmcnt<(NS > 3 ? LOADS * (NS - 3) : 0) + EXTRA>();
-    else
-      wait_vmcnt<(NS > 3 ? LOADS * (NS - 3) : 0)>();
-  } else {
-    if (extra)
-      wait_vmcnt<EXTRA>();
-    else
-      wait_vmcnt<0>();
+      wait_vmcnt<LOADS * LATER>();
+  } else if constexpr (LATER > 0) {
+    wait_slab<LOADS, LATER - 1, EXTRA>(ahead, extra);
   }
 }
 
@@ -224,16 +235,24 @@ template <>
 struct Path<false> {
   typedef bf16x8 frag;
   typedef f32x16 acc;
+  typedef f32x4 acc4;
   static __device__ __forceinline__ acc mfma(frag w, frag a, acc c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, a, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ acc4 mfma16(frag w, frag a, acc4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, c, 0, 0, 0);
   }
 };
 template <>
 struct Path<true> {
   typedef i32x4 frag;
   typedef i32x16 acc;
+  typedef i32x4 acc4;
   static __device__ __forceinline__ acc mfma(frag w, frag a, acc c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(w, a, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ acc4 mfma16(frag w, frag a, acc4 c) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(w, a, c, 0, 0, 0);
   }
 };
 
@@ -241,7 +260,7 @@ struct Path<true> {
 // (else fp32); I8: the int8 datapath; RAW (int8 only): store the int32
 // accumulators, no bias, scales or activation.
 template <int BM, int BN, int WGM, int WGN, int NS, int EPI, bool RES, bool CBF, bool I8,
-          bool RAW, int RB = 64>
+          bool RAW, int RB = 64, bool M16 = false>
 __device__ __forceinline__ void gemm_lds_body(
     const void *__restrict__ A, int64_t lda, const void *__restrict__ Wt, int M, int N, int K,
     const float *__restrict__ bias, const float *residual, void *C, int64_t ldc, int tiles_m,
@@ -252,6 +271,8 @@ __device__ __forceinline__ void gemm_lds_body(
   using PT = Path<I8>;
   typedef typename PT::frag frag_t;
   typedef typename PT::acc acc_t;
+  typedef typename PT::acc4 acc4_t;
+  static_assert(!M16 || EPI < 8 || (EPI & EPI_NARROW_C), "16 x 16 tiles: not the gated FFN");
   static_assert(I8 || !RAW, "RAW is the int8 datapath's");
   static_assert(!RAW || (EPI == 0 && !RES && !CBF), "RAW stores the accumulators as they are");
   constexpr int TM = Cfg::TM, TN = Cfg::TN, ESZ = Cfg::ESZ;
@@ -355,16 +376,19 @@ __device__ __forceinline__ void gemm_lds_body(
   // Issue the loads of slab is_s, then advance the cursor.
   uint32_t is_slot = 0;  // byte offset of slot is_s % NS
   uint64_t is_kb = 0;    // byte depth of slab is_kt
-  auto issue = [&]() {
-    const int ti = is_ti, kt = is_kt, n0 = is_n0, m0 = is_m0;
+  auto issue_loads = [&](int k0, int k1) {  // the slab's loads k0 .. k1 - 1
     const uint32_t slot = lds0 + is_slot;
 #pragma unroll
     for (int k = 0; k < Cfg::LOADS_HI; ++k) {
+      if (k < k0 || k >= k1) continue;
       const int p = wave + Cfg::NW * k;  // wave-uniform
       if (k < Cfg::LOADS_LO || p < Cfg::PIECES)
         dma16s((SPLIT ? (is_a(k) ? abase : bbase) : pbase[k]) + is_kb, poff[k],
                slot + (uint32_t)(p * 1024));
     }
+  };
+  auto issue_end = [&]() {
+    const int ti = is_ti, kt = is_kt, n0 = is_n0, m0 = is_m0;
     // Epilogue vectors, on a tile's first slab: lanes 0 .. BIAS_PER_WAVE/4 - 1
     // move 16 bytes each of the columns from n0 + wave * BIAS_PER_WAVE (clamped
     // in bounds; a column >= N is never stored); for int8, lanes
@@ -400,39 +424,75 @@ __device__ __forceinline__ void gemm_lds_body(
       }
     }
   };
+  auto issue = [&]() {
+    issue_loads(0, Cfg::LOADS_HI);
+    issue_end();
+  };
 
   constexpr bool SAME_LOADS_P = Cfg::LOADS_HI == Cfg::LOADS_LO;
   static_assert(Cfg::LOADS_HI * (NS - 1) < 64, "vmcnt holds at most 63");
-  acc_t acc[TN][TM];
+  // Accumulators per 32 x 32 block: one 32 x 32 MFMA tile, or (M16) four
+  // 16 x 16 ones, tile q = 2 * (row half) + (column half).
+  acc_t acc[M16 ? 1 : TN][M16 ? 1 : TM];
+  acc4_t acc4[M16 ? TN : 1][M16 ? TM : 1][4];
+  auto clear_acc = [&]() {
+    if constexpr (M16) {
 #pragma unroll
-  for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][i][r] = 0;
+          for (int r = 0; r < 16; ++r) acc4[j][i][r >> 2][r & 3] = 0;
+    } else {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[j][i][r] = 0;
+    }
+  };
+  clear_acc();
+  auto acc_at = [&](int j, int i, int r) {
+    if constexpr (M16)
+      return acc4[j][i][r >> 2][r & 3];
+    else
+      return acc[j][i][r];
+  };
+  // A lane's accumulator elements 4q .. 4q + 3 of a block are row rq(q),
+  // columns cq(q) .. cq(q) + 3 of the block.
+  auto rq = [&](int q) { return M16 ? (q >> 1) * 16 + (lane & 15) : li; };
+  auto cq = [&](int q) { return M16 ? (q & 1) * 16 + (lane >> 4) * 4 : q * 8 + g * 4; };
   // Accumulator element r of block (j, i) as the epilogue reads it: as it is,
   // or (NC) rounded to bf16 first.
   auto accf = [&](int j, int i, int r) -> float {
     if constexpr (I8) {
-      if constexpr (NC) return bf2f(i32_to_bf16((int)acc[j][i][r]));
-      return (float)acc[j][i][r];
+      if constexpr (NC) return bf2f(i32_to_bf16((int)acc_at(j, i, r)));
+      return (float)acc_at(j, i, r);
     } else {
-      if constexpr (NC) return bf2f(f2bf(acc[j][i][r]));
-      return acc[j][i][r];
+      if constexpr (NC) return bf2f(f2bf(acc_at(j, i, r)));
+      return acc_at(j, i, r);
     }
   };
 
   // Fragment addressing: at k-step kk lane (row li, k-half g) reads logical
   // chunk 2*kk + g of its row, at its swizzled position (rows 32*x + li all
   // share li's swizzle).
-  constexpr int KS = Cfg::KSTEPS;
-  static_assert(KS % 2 == 0, "the last k-step of a slab is in set 1");
+  // (M16: k-steps of 64 bytes; lane (row l % 16, quarter l / 16) reads chunk
+  // 4*kk + l / 16 of rows 16*x + l % 16.)
+  constexpr int KS = M16 ? Cfg::KSTEPS / 2 : Cfg::KSTEPS;
+  static_assert(M16 || KS % 2 == 0, "the last k-step of a slab is in set 1");
   int pos[KS];
 #pragma unroll
-  for (int kk = 0; kk < KS; ++kk) pos[kk] = chunk_pos<RB>(2 * kk + g, li) * 16;
-  const int rowA = (wm * Cfg::WM + li) * RB, rowB = (wn * Cfg::WN + li) * RB;
+  for (int kk = 0; kk < KS; ++kk)
+    pos[kk] = M16 ? chunk_pos<RB>(4 * kk + (lane >> 4), lane & 15) * 16
+                  : chunk_pos<RB>(2 * kk + g, li) * 16;
+  const int frow = M16 ? lane & 15 : li;
+  const int rowA = (wm * Cfg::WM + frow) * RB, rowB = (wn * Cfg::WN + frow) * RB;
 
-  frag_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
+  // One k-step's fragments per set, or (M16) a whole slab's.
+  constexpr int FA = M16 ? 2 * KS * TM : TM, FB = M16 ? 2 * KS * TN : TN;
+  frag_t fa0[FA], fb0[FB], fa1[FA], fb1[FB];
   // Reads in the order the MFMAs consume them: fb[0], fa[0..TM), fb[1..TN);
   // read x of that order for x in [x0, x1).
   auto read_part = [&](uint32_t soff, int pos, frag_t *fa, frag_t *fb, int x0, int x1) {
@@ -451,6 +511,26 @@ __device__ __forceinline__ void gemm_lds_body(
   auto read_set = [&](uint32_t soff, int pos, frag_t *fa, frag_t *fb) {
     read_part(soff, pos, fa, fb, 0, TM + TN);
   };
+  // M16: k-step kk of a slab into (MFMAs from) a whole-slab set.
+  auto read16 = [&](uint32_t soff, int kk, frag_t *fa, frag_t *fb) {
+    const uint8_t *slot = smem + soff + pos[kk];
+#pragma unroll
+    for (int x = 0; x < 2 * TN; ++x)
+      fb[kk * 2 * TN + x] = *(const frag_t *)(slot + Cfg::A_BYTES + rowB + x * 16 * RB);
+#pragma unroll
+    for (int x = 0; x < 2 * TM; ++x)
+      fa[kk * 2 * TM + x] = *(const frag_t *)(slot + rowA + x * 16 * RB);
+  };
+  auto mfma16_set = [&](int kk, const frag_t *fa, const frag_t *fb) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          acc4[j][i][q] = PT::mfma16(fb[kk * 2 * TN + 2 * j + (q & 1)],
+                                     fa[kk * 2 * TM + 2 * i + (q >> 1)], acc4[j][i][q]);
+  };
   auto mfma_set = [&](const frag_t *fa, const frag_t *fb) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
@@ -458,14 +538,20 @@ __device__ __forceinline__ void gemm_lds_body(
       for (int i = 0; i < TM; ++i) acc[j][i] = PT::mfma(fb[j], fa[i], acc[j][i]);
   };
   // MFMAs and the LDS reads of the other set, one read after each of the
-  // first TM + TN MFMAs.
+  // first TM + TN MFMAs (a wave tile with fewer MFMAs than reads issues its
+  // reads first: they are what the next k-step waits for).
   auto interleave = []() {
+    if constexpr (TM * TN >= TM + TN) {
 #pragma unroll
-    for (int x = 0; x < TM + TN; ++x) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
+      for (int x = 0; x < TM + TN; ++x) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - (TM + TN), 0);
+    } else {
+      __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, TM * TN, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - (TM + TN), 0);
   };
 
   // The epilogue of a bf16 C without a residual, block by block (k = j * TM
@@ -533,9 +619,9 @@ __device__ __forceinline__ void gemm_lds_body(
           const int cl = wn * Cfg::WN + ja * 32;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            b[q] = has_bias ? *(const float4 *)(bl + cl + q * 8 + g * 4)
+            b[q] = has_bias ? *(const float4 *)(bl + cl + cq(q))
                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (I8) w[q] = *(const float4 *)(wsl + cl + q * 8 + g * 4);
+            if (I8) w[q] = *(const float4 *)(wsl + cl + cq(q));
           }
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
@@ -561,14 +647,14 @@ __device__ __forceinline__ void gemm_lds_body(
           const int cl = wn * Cfg::WN + j * 32;  // tile-local first column
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            b[q] = has_bias ? *(const float4 *)(bl + cl + q * 8 + g * 4)
+            b[q] = has_bias ? *(const float4 *)(bl + cl + cq(q))
                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (I8) w[q] = *(const float4 *)(wsl + cl + q * 8 + g * 4);
+            if (I8) w[q] = *(const float4 *)(wsl + cl + cq(q));
           }
         }
-        const float sa = I8 ? sal[wm * Cfg::WM + i * 32 + li] : 0.0f;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
+          const float sa = I8 ? sal[wm * Cfg::WM + i * 32 + rq(q)] : 0.0f;
           const float bb[4] = {b[q].x, b[q].y, b[q].z, b[q].w};
           const float ww[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
           float v[4];
@@ -581,7 +667,8 @@ __device__ __forceinline__ void gemm_lds_body(
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        *(uint2 *)(stg + li * 64 + ((q ^ ((li >> 2) & 3)) * 16 + g * 8)) =
+        *(uint2 *)(stg + rq(q) * 64 +
+                   (((cq(q) >> 3) ^ ((rq(q) >> 2) & 3)) * 16 + ((cq(q) >> 2) & 1) * 8)) =
             make_uint2(pk[2 * q], pk[2 * q + 1]);
       if (k > 0) store(k - 1, wv);
 #pragma unroll
@@ -633,38 +720,37 @@ __device__ __forceinline__ void gemm_lds_body(
       if (k + 1 < TM * TN) load_res(k + 1, rnext);
       const int rbase = m0 + wm * Cfg::WM + i * 32;
       const int cl = wn * Cfg::WN + j * 32;
-      const float sa = I8 ? sal[wm * Cfg::WM + i * 32 + li] : 0.0f;
-      float4 vq[4];  // columns 8q + 4g .. + 3 of row li
+      float4 vq[4];  // columns cq(q) .. + 3 of row rq(q)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float4 b = has_bias ? *(const float4 *)(bl + cl + q * 8 + g * 4)
+        const float sa = I8 ? sal[wm * Cfg::WM + i * 32 + rq(q)] : 0.0f;
+        const float4 b = has_bias ? *(const float4 *)(bl + cl + cq(q))
                                   : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float4 v;
         if (I8) {
-          const float4 w = *(const float4 *)(wsl + cl + q * 8 + g * 4);
+          const float4 w = *(const float4 *)(wsl + cl + cq(q));
           v.x = gemm_epilogue(
-              __builtin_fmaf(__fmul_rn((float)acc[j][i][q * 4 + 0], sa), w.x, b.x), EPB);
+              __builtin_fmaf(__fmul_rn((float)acc_at(j, i, q * 4 + 0), sa), w.x, b.x), EPB);
           v.y = gemm_epilogue(
-              __builtin_fmaf(__fmul_rn((float)acc[j][i][q * 4 + 1], sa), w.y, b.y), EPB);
+              __builtin_fmaf(__fmul_rn((float)acc_at(j, i, q * 4 + 1), sa), w.y, b.y), EPB);
           v.z = gemm_epilogue(
-              __builtin_fmaf(__fmul_rn((float)acc[j][i][q * 4 + 2], sa), w.z, b.z), EPB);
+              __builtin_fmaf(__fmul_rn((float)acc_at(j, i, q * 4 + 2), sa), w.z, b.z), EPB);
           v.w = gemm_epilogue(
-              __builtin_fmaf(__fmul_rn((float)acc[j][i][q * 4 + 3], sa), w.w, b.w), EPB);
+              __builtin_fmaf(__fmul_rn((float)acc_at(j, i, q * 4 + 3), sa), w.w, b.w), EPB);
         } else {
-          v.x = gemm_epilogue(acc[j][i][q * 4 + 0] + b.x, EPB);
-          v.y = gemm_epilogue(acc[j][i][q * 4 + 1] + b.y, EPB);
-          v.z = gemm_epilogue(acc[j][i][q * 4 + 2] + b.z, EPB);
-          v.w = gemm_epilogue(acc[j][i][q * 4 + 3] + b.w, EPB);
+          v.x = gemm_epilogue(acc_at(j, i, q * 4 + 0) + b.x, EPB);
+          v.y = gemm_epilogue(acc_at(j, i, q * 4 + 1) + b.y, EPB);
+          v.z = gemm_epilogue(acc_at(j, i, q * 4 + 2) + b.z, EPB);
+          v.w = gemm_epilogue(acc_at(j, i, q * 4 + 3) + b.w, EPB);
         }
         vq[q] = v;
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        if ((li >> 4) == h) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            *(float4 *)(stg + (li & 15) * STG_ROWB + (q * 8 + g * 4) * 4) = vq[q];
-        }
+        for (int q = 0; q < 4; ++q)
+          if ((rq(q) >> 4) == h)
+            *(float4 *)(stg + (rq(q) & 15) * STG_ROWB + cq(q) * 4) = vq[q];
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int part = 0; part < 2; ++part) {
@@ -706,8 +792,6 @@ __device__ __forceinline__ void gemm_lds_body(
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int rbase = m0 + wm * Cfg::WM + i * 32;
-      float sa = 0.0f;
-      if (I8 && !RAW) sa = sal[wm * Cfg::WM + i * 32 + li];
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const int cl = wn * Cfg::WN + j * 32;  // tile-local first column
@@ -720,16 +804,17 @@ __device__ __forceinline__ void gemm_lds_body(
         // added before the one rounding).
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
+          const float sa = I8 && !RAW ? sal[wm * Cfg::WM + i * 32 + rq(q)] : 0.0f;
           float4 v;
           if (RAW) {
-            v.x = __int_as_float((int)acc[j][i][q * 4 + 0]);
-            v.y = __int_as_float((int)acc[j][i][q * 4 + 1]);
-            v.z = __int_as_float((int)acc[j][i][q * 4 + 2]);
-            v.w = __int_as_float((int)acc[j][i][q * 4 + 3]);
+            v.x = __int_as_float((int)acc_at(j, i, q * 4 + 0));
+            v.y = __int_as_float((int)acc_at(j, i, q * 4 + 1));
+            v.z = __int_as_float((int)acc_at(j, i, q * 4 + 2));
+            v.w = __int_as_float((int)acc_at(j, i, q * 4 + 3));
           } else if (I8) {
-            const float4 b = has_bias ? *(const float4 *)(bl + cl + q * 8 + g * 4)
+            const float4 b = has_bias ? *(const float4 *)(bl + cl + cq(q))
                                       : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const float4 w = *(const float4 *)(wsl + cl + q * 8 + g * 4);
+            const float4 w = *(const float4 *)(wsl + cl + cq(q));
             v.x = gemm_epilogue(__builtin_fmaf(__fmul_rn(accf(j, i, q * 4 + 0), sa), w.x, b.x),
                                 EPB);
             v.y = gemm_epilogue(__builtin_fmaf(__fmul_rn(accf(j, i, q * 4 + 1), sa), w.y, b.y),
@@ -739,7 +824,7 @@ __device__ __forceinline__ void gemm_lds_body(
             v.w = gemm_epilogue(__builtin_fmaf(__fmul_rn(accf(j, i, q * 4 + 3), sa), w.w, b.w),
                                 EPB);
           } else {
-            const float4 b = *(const float4 *)(bl + cl + q * 8 + g * 4);
+            const float4 b = *(const float4 *)(bl + cl + cq(q));
             v.x = gemm_epilogue(accf(j, i, q * 4 + 0) + b.x, EPB);
             v.y = gemm_epilogue(accf(j, i, q * 4 + 1) + b.y, EPB);
             v.z = gemm_epilogue(accf(j, i, q * 4 + 2) + b.z, EPB);
@@ -747,9 +832,10 @@ __device__ __forceinline__ void gemm_lds_body(
           }
           if (STG_BF) {
             const uint2 w = make_uint2(pack_bf2_hw(v.x, v.y), pack_bf2_hw(v.z, v.w));
-            *(uint2 *)(stg + li * 64 + ((q ^ ((li >> 2) & 3)) * 16 + g * 8)) = w;
+            *(uint2 *)(stg + rq(q) * 64 +
+                       (((cq(q) >> 3) ^ ((rq(q) >> 2) & 3)) * 16 + ((cq(q) >> 2) & 1) * 8)) = w;
           } else {
-            *(float4 *)(stg + li * STG_ROWB + (q * 8 + g * 4) * 4) = v;
+            *(float4 *)(stg + rq(q) * STG_ROWB + cq(q) * 4) = v;
           }
         }
         asm volatile("" ::: "memory");
@@ -848,7 +934,12 @@ __device__ __forceinline__ void gemm_lds_body(
   }
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  read_set(0, pos[0], fa0, fb0);
+  if constexpr (M16) {
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) read16(0, kk, fa0, fb0);
+  } else {
+    read_set(0, pos[0], fa0, fb0);
+  }
 
   // An epilogue issues EPI_STORES global stores per wave (one per staged row
   // group of each 32 x 32 block) when its tile lies wholly inside C, where
@@ -863,25 +954,10 @@ __device__ __forceinline__ void gemm_lds_body(
   int epi_left = 0;
   int ep_kt = 0, ep_ti = 0;  // tile and depth of slab s
   uint32_t rd_slot = 0;      // byte offset of slab s's slot
-  for (int s = 0; s < nslab; ++s) {
-    // k-steps 0 .. KS-2 of slab s: each one's MFMAs run while the next
-    // k-step's fragments are read into the other set.
-#pragma unroll
-    for (int kk = 0; kk + 1 < KS; ++kk) {
-      if (kk % 2 == 0) {
-        mfma_set(fa0, fb0);
-        read_set(rd_slot, pos[kk + 1], fa1, fb1);
-      } else {
-        mfma_set(fa1, fb1);
-        read_set(rd_slot, pos[kk + 1], fa0, fb0);
-      }
-      interleave();
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // Every read of slab s is now issued. Wait for them and for this wave's
-    // loads of slab s + 1 (the slabs issued after it, at most NS - 2, may stay
-    // in flight), then meet: slab s + 1 is in LDS and slot s % NS is free.
-    const uint32_t nx_slot = rd_slot + Cfg::SLOT == NS * Cfg::SLOT ? 0 : rd_slot + Cfg::SLOT;
+  // Wait for this wave's LDS reads of slab s and for its loads of slab s + 1
+  // (the slabs issued after it, at most NS - 2, may stay in flight), then
+  // meet the other waves.
+  auto meet = [&](int s) {
     const int ahead = nslab - 2 - s;
     const bool stores_young = EPI_STORES > 0 && epi_left > 0;
     if (ahead >= NS - 2 && !stores_young) {
@@ -890,47 +966,17 @@ __device__ __forceinline__ void gemm_lds_body(
       else
         wait_vmcnt<Cfg::LOADS_LO *(NS - 2)>();
     } else if (SAME_LOADS || wave < Cfg::NHI) {
-      wait_slab<Cfg::LOADS_HI, NS, EPI_STORES>(ahead, stores_young);
+      wait_slab<Cfg::LOADS_HI, NS - 2, EPI_STORES>(ahead, stores_young);
     } else {
-      wait_slab<Cfg::LOADS_LO, NS, EPI_STORES>(ahead, stores_young);
+      wait_slab<Cfg::LOADS_LO, NS - 2, EPI_STORES>(ahead, stores_young);
     }
     if (epi_left > 0) --epi_left;
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    // The last k-step of slab s (set 1: KS is even); k-step 0 of slab s + 1
-    // is read meanwhile, in consumption order (after the last slab, slab s
-    // again: in bounds, unused): the first TM reads beside the j = 0 MFMAs,
-    // the rest after the loads of slab s + NS are issued -- those keep the
-    // matrix pipe busy while the scalar unit addresses the loads.
-    const uint32_t rs = s + 1 < nslab ? nx_slot : rd_slot;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) acc[0][i] = PT::mfma(fb1[0], fa1[i], acc[0][i]);
-    read_part(rs, pos[0], fa0, fb0, 0, TM);
-#pragma unroll
-    for (int x = 0; x < TM; ++x) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + NS < nslab) issue();  // slab s + NS
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 1; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i) acc[j][i] = PT::mfma(fb1[j], fa1[i], acc[j][i]);
-    read_part(rs, pos[0], fa0, fb0, TM, TM + TN);
-    {
-      constexpr int NM = TM * (TN - 1), NR = TN, NP = NM < NR ? NM : NR;
-#pragma unroll
-      for (int x = 0; x < NP; ++x) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
-      if (NM > NP) __builtin_amdgcn_sched_group_barrier(0x008, NM - NP, 0);
-      if (NR > NP) __builtin_amdgcn_sched_group_barrier(0x100, NR - NP, 0);
-    }
-    rd_slot = nx_slot;
+  };
+  // Slab s is consumed: at the end of a tile, its epilogue.
+  auto finish = [&]() {
     if (++ep_kt == nk) {
       ep_kt = 0;
       {
@@ -939,12 +985,96 @@ __device__ __forceinline__ void gemm_lds_body(
         epi_left = (m0 + BM <= M && n0 + BN <= N) ? NS - 1 : 0;
       }
       epilogue(ep_ti++);
+      clear_acc();
+    }
+  };
+  if constexpr (M16) {
+    // Whole-slab sets: while slab s's MFMAs run from one register set, slab
+    // s + 1's fragments are read into the other and slab s + NS is issued, a
+    // share of both behind each k-step's MFMAs.
+    auto body = [&](auto fill, uint32_t rs, frag_t *fa, frag_t *fb, frag_t *na, frag_t *nb) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int kk = 0; kk < KS; ++kk) {
+        mfma16_set(kk, fa, fb);
+        read16(rs, kk, na, nb);
+        if (decltype(fill)::value)
+          issue_loads(kk * Cfg::LOADS_HI / KS, (kk + 1) * Cfg::LOADS_HI / KS);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto step = [&](int s, frag_t *fa, frag_t *fb, frag_t *na, frag_t *nb) {
+      const uint32_t nx_slot = rd_slot + Cfg::SLOT == NS * Cfg::SLOT ? 0 : rd_slot + Cfg::SLOT;
+      meet(s);
+      __builtin_amdgcn_sched_barrier(0);
+      // (after the last slab, slab s again: in bounds, unused)
+      if (s + NS < nslab) {
+        body(std::true_type{}, nx_slot, fa, fb, na, nb);
+        issue_end();
+      } else {
+        body(std::false_type{}, s + 1 < nslab ? nx_slot : rd_slot, fa, fb, na, nb);
+      }
+      rd_slot = nx_slot;
+      finish();
+    };
+    for (int s = 0; s < nslab; s += 2) {
+      step(s, fa0, fb0, fa1, fb1);
+      if (s + 1 < nslab) step(s + 1, fa1, fb1, fa0, fb0);
+    }
+  } else {
+    for (int s = 0; s < nslab; ++s) {
+      // k-steps 0 .. KS-2 of slab s: each one's MFMAs run while the next
+      // k-step's fragments are read into the other set.
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+      for (int kk = 0; kk + 1 < KS; ++kk) {
+        if (kk % 2 == 0) {
+          mfma_set(fa0, fb0);
+          read_set(rd_slot, pos[kk + 1], fa1, fb1);
+        } else {
+          mfma_set(fa1, fb1);
+          read_set(rd_slot, pos[kk + 1], fa0, fb0);
+        }
+        interleave();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // Every read of slab s is now issued. Wait for them and for this wave's
+      // loads of slab s + 1 (the slabs issued after it, at most NS - 2, may stay
+      // in flight), then meet: slab s + 1 is in LDS and slot s % NS is free.
+      const uint32_t nx_slot = rd_slot + Cfg::SLOT == NS * Cfg::SLOT ? 0 : rd_slot + Cfg::SLOT;
+      meet(s);
+      // The last k-step of slab s (set 1: KS is even); k-step 0 of slab s + 1
+      // is read meanwhile, in consumption order (after the last slab, slab s
+      // again: in bounds, unused): the first TM reads beside the j = 0 MFMAs,
+      // the rest after the loads of slab s + NS are issued -- those keep the
+      // matrix pipe busy while the scalar unit addresses the loads.
+      const uint32_t rs = s + 1 < nslab ? nx_slot : rd_slot;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[j][i][r] = 0;
+      for (int i = 0; i < TM; ++i) acc[0][i] = PT::mfma(fb1[0], fa1[i], acc[0][i]);
+      read_part(rs, pos[0], fa0, fb0, 0, TM);
+#pragma unroll
+      for (int x = 0; x < TM; ++x) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + NS < nslab) issue();  // slab s + NS
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 1; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[j][i] = PT::mfma(fb1[j], fa1[i], acc[j][i]);
+      read_part(rs, pos[0], fa0, fb0, TM, TM + TN);
+      {
+        constexpr int NM = TM * (TN - 1), NR = TN, NP = NM < NR ? NM : NR;
+#pragma unroll
+        for (int x = 0; x < NP; ++x) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        if constexpr (NM > NP) __builtin_amdgcn_sched_group_barrier(0x008, NM - NP, 0);
+        if constexpr (NR > NP) __builtin_amdgcn_sched_group_barrier(0x100, NR - NP, 0);
+      }
+      rd_slot = nx_slot;
+      finish();
     }
   }
 }

@@ -1,0 +1,91 @@
+"""The GEMM's 16 x 16 MFMA forms and its paired 128 x 128 tile, at the sizes
+where a tile, a slab ring or a wave's share of either can go wrong.
+
+Every tile runs the same chain of products over K for each element of C, so a
+row's bits do not depend on the row count that chose the tile: each product is
+compared bit for bit with the same rows of a 20,000-row one, which the large
+tiles serve (their own tests hold those to the oracle), and a part of it with
+the oracle's gemm_nt at that test's bounds."""
+import numpy as np
+import pytest
+
+import mxenc
+from mxenc import from_bf16_bits, to_bf16_bits
+from orc import P
+
+pytestmark = pytest.mark.gpu
+
+NONE, POLY, ERF = mxenc.MX_EPI_NONE, mxenc.MX_EPI_GELU_POLY, mxenc.MX_EPI_GELU_ERF
+BIG = 20000
+
+CASES = [
+    # M, K, N, epilogue, C dtype, residual, expected kernel
+    (1, 384, 1152, NONE, np.uint16, False, "lds_64x64x128_w32x32_ns3_mfma16"),  # one row
+    (19, 1536, 384, NONE, np.uint16, False, "lds_64x64x128_w32x32_ns3_mfma16"),
+    (65, 768, 3072, ERF, np.uint16, False, "lds_64x64x128_w32x32_ns3_mfma16"),  # a row over
+    (127, 3072, 768, NONE, np.float32, True, "lds_64x64x128_w32x32_ns3_mfma16"),
+    (200, 1920, 640, POLY, np.float32, True, "lds_64x64x128_w32x32_ns3_mfma16"),  # odd slabs
+    (300, 768, 768, NONE, np.float32, False, "lds_64x64x128_w32x32_ns3_mfma16"),
+    (1500, 1024, 1024, NONE, np.uint16, False, "lds_64x64x128_w32x32_ns2_mfma16"),
+    (1473, 768, 768, POLY, np.float32, True, "lds_64x64x128_w32x32_ns2_mfma16"),
+    (31, 256, 64, ERF, np.uint16, False, "lds_64x64x128_w32x32_ns2_mfma16"),  # two slabs
+    (333, 448, 448, POLY, np.uint16, False, "lds_64x64x64_w32x32_ns4_mfma16"),  # K % 128 = 64
+    (63, 320, 1344, NONE, np.float32, True, "lds_64x64x64_w32x32_ns4_mfma16"),
+    (3000, 1280, 1280, NONE, np.float32, True, "lds_128x128x64_w64x32_ns4_mfma16"),
+    (1999, 256, 1288, ERF, np.uint16, False, "lds_128x128"),  # ragged M and N
+    (3940, 5120, 1280, NONE, np.float32, True, "lds_128x128x64_w64x64_ns2"),
+    (3940, 5120, 1280, POLY, np.uint16, False, "lds_128x128x64_w64x64_ns2"),
+]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = mxenc.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("M,K,N,epi,cdt,res,plan", CASES)
+def test_small_tiles(ctx, orc, M, K, N, epi, cdt, res, plan):
+    print("case", M, K, N, epi, cdt, res, flush=True)
+    dt = mxenc.MX_BF16 if cdt == np.uint16 else mxenc.MX_F32
+    L = mxenc.lib()
+    assert L.mx_gemm_plan_for(M, N, K, dt, int(res), 0).decode().startswith(plan)
+    rng = np.random.default_rng(M + K + N)
+    A = np.zeros((BIG, K), np.uint16)
+    A[:M] = to_bf16_bits(rng.standard_normal((M, K)).astype(np.float32))
+    W = to_bf16_bits((rng.standard_normal((K, N)) * 0.05).astype(np.float32))
+    bias = (rng.standard_normal(N) * 0.1).astype(np.float32)
+    R = rng.standard_normal((BIG, N)).astype(np.float32) if res else None
+    dW, db = ctx.put(np.ascontiguousarray(W.T)), ctx.put(bias)
+
+    def product(rows):
+        dA = ctx.put(A[:rows])
+        # one row more than C has: nothing is written past the last
+        dC = ctx.put(R[:rows]) if res else ctx.put(np.zeros((rows + 1, N), cdt))
+        mxenc.gemm_wt(ctx, dA, rows, K, K, dW, N, db, epi, dC if res else None, dC, N)
+        return dC.host()
+
+    got, big = product(M), product(BIG)
+    if not res:
+        assert not got[M].any()
+    got = got[:M]
+    assert np.array_equal(got.view(np.uint8), big[:M].view(np.uint8))
+
+    rows = np.unique(np.concatenate([np.arange(min(M, 64)), np.arange(max(0, M - 64), M)]))
+    want = np.empty((rows.size, N), np.float32)
+    Af = np.ascontiguousarray(from_bf16_bits(A[rows]))
+    Wf = np.ascontiguousarray(from_bf16_bits(W))
+    orc.orc_gemm_nt(P(Af), rows.size, P(Wf), K, N, P(bias), P(want))
+    if epi == POLY:
+        orc.orc_gelu_poly_inplace(P(want), want.size)
+    elif epi == ERF:
+        orc.orc_gelu_erf_inplace(P(want), want.size)
+    if res:
+        want += R[rows]
+    scale = np.max(np.abs(want))
+    if cdt == np.uint16:
+        g = from_bf16_bits(got[rows])
+        assert np.max(np.abs(g - want) / (np.abs(want) + 1e-3 * scale)) < 1e-2
+    else:
+        assert np.max(np.abs(got[rows] - want)) / scale < 1e-5
