@@ -55,7 +55,7 @@ def kernel_name(plan, epi, res, cbf, i8=False):
     runs, e.g. lds_256x256x64_w64x128_ns2_persistent (bf16) ->
     gemm_lds_k<256, 256, 4, 2, 2, epi, res, cbf, 128>; the last argument is the
     slab row in bytes (slab K times the element size). gemm_i8_k<...> on the
-    int8 datapath."""
+    int8 datapath; gemm_lds16_k and gemm_i8_16_k for an mfma16 plan."""
     if not plan.startswith("lds_"):
         return "gemm_bf16_k<128, 128, 64, 64, 64>"
     tile, wave, ns = plan.split("_")[1:4]
@@ -63,10 +63,11 @@ def kernel_name(plan, epi, res, cbf, i8=False):
     wm, wn = (int(x) for x in wave[1:].split("x"))
     rb = bk * (1 if i8 else 2)
     b = lambda v: "true" if v else "false"  # noqa: E731
+    m16 = "_mfma16" in plan
     if i8:
-        return (f"gemm_i8_k<{bm}, {bn}, {bm // wm}, {bn // wn}, {int(ns[2:])}, {epi}, {b(res)}, "
+        return (f"gemm_i8_{'16_' if m16 else ''}k<{bm}, {bn}, {bm // wm}, {bn // wn}, {int(ns[2:])}, {epi}, {b(res)}, "
                 f"{1 if cbf else 0}, {rb}>")
-    return (f"gemm_lds_k<{bm}, {bn}, {bm // wm}, {bn // wn}, {int(ns[2:])}, {epi}, {b(res)}, "
+    return (f"gemm_lds{'16' if m16 else ''}_k<{bm}, {bn}, {bm // wm}, {bn // wn}, {int(ns[2:])}, {epi}, {b(res)}, "
             f"{b(cbf)}, {rb}>")
 
 

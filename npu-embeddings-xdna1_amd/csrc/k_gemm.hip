@@ -359,12 +359,14 @@ const char *gemm_plan_name(int64_t M, int64_t N, int64_t K, bool c_bf16, bool re
     a.c_dtype = c_bf16 ? 1 : 0;
     a.residual = residual ? aligned_probe : nullptr;
     const bool deep = gemm_i8_deep(a);
-    switch (gemm_lds_tile(M, N, deep)) {
+    switch (gemm_i8_tile(a)) {
       case 0:
         return deep ? "lds_256x256x128_w64x128_ns2_persistent"
                     : "lds_256x256x64_w128x64_ns3_persistent";
       case 1: return "lds_256x192x64_w64x96_ns4_persistent";
       case 2: return "lds_128x256x64_w64x64_ns4_persistent";
+      case 4: return "lds_128x128x128_w64x32_ns3_mfma16_persistent";
+      case 5: return "lds_64x64x256_w32x32_ns3_mfma16_persistent";
       default: return "lds_128x128x64_w64x64_ns4_persistent";
     }
   }

@@ -167,6 +167,8 @@ struct GemmI8Args {
 hipError_t gemm_i8(const GemmI8Args &a, hipStream_t s);
 // Whether the 256 x 256 tile runs on 128-byte slabs for this call.
 bool gemm_i8_deep(const GemmI8Args &a);
+// The tile of a call that is not narrowed (k_gemm_i8.hip).
+int gemm_i8_tile(const GemmI8Args &a);
 
 // quantise_a_int8 over rows of K (k_quant.hip): a fp32 or bf16 (row stride
 // lda), ias [K] -> q int8 (row stride ldq) and a_scale [rows]. K % 4 == 0,

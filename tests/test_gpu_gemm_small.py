@@ -89,3 +89,61 @@ def test_small_tiles(ctx, orc, M, K, N, epi, cdt, res, plan):
         assert np.max(np.abs(g - want) / (np.abs(want) + 1e-3 * scale)) < 1e-2
     else:
         assert np.max(np.abs(got[rows] - want)) / scale < 1e-5
+
+
+I8_CASES = [
+    # M, K, N, epilogue, C dtype, residual, expected kernel
+    (1, 768, 2304, NONE, np.uint16, False, "lds_64x64x256_w32x32_ns3_mfma16"),  # one row
+    (65, 1024, 4096, POLY, np.float32, False, "lds_64x64x256_w32x32_ns3_mfma16"),  # a row over
+    (300, 3072, 768, NONE, np.float32, False, "lds_64x64x256_w32x32_ns3_mfma16"),
+    (127, 1280, 1280, ERF, np.float32, True, "lds_64x64x256_w32x32_ns3_mfma16"),
+    (300, 384, 1152, NONE, np.float32, False, "lds_128x128x128_w64x32_ns3_mfma16"),  # three slabs
+    (4099, 3072, 768, NONE, np.float32, False, "lds_128x128x128_w64x32_ns3_mfma16"),
+    (1000, 896, 1000, POLY, np.uint16, False, "lds_128x128x128_w64x32_ns3_mfma16"),  # ragged N
+    (999, 1152, 1152, NONE, np.float32, True, "lds_128x128x128_w64x32_ns3_mfma16"),
+]
+
+
+@pytest.mark.parametrize("M,K,N,epi,cdt,res,plan", I8_CASES)
+def test_small_tiles_i8(ctx, orc, M, K, N, epi, cdt, res, plan):
+    """The int32 product is exact, so the dequantised result is the host's bit
+    for bit (the exact-erf GELU and the residual's sum to one rounding)."""
+    print("case", M, K, N, epi, cdt, res, flush=True)
+    dt = mxenc.MX_BF16 if cdt == np.uint16 else mxenc.MX_F32
+    L = mxenc.lib()
+    assert L.mx_gemm_plan_for(M, N, K, dt, int(res), 1).decode().startswith(plan)
+    rng = np.random.default_rng(M + K + N)
+    A = rng.integers(-127, 128, (M, K)).astype(np.int8)
+    W = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    sa = rng.uniform(1e-4, 1e-2, M).astype(np.float32)
+    ws = rng.uniform(1e-4, 1e-2, N).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    R = rng.standard_normal((M, N)).astype(np.float32) if res else None
+    slot = mxenc.stage_weight_i8(ctx, W, ws, np.ones(K, np.float32))
+    # a row more than C has: nothing is written past the last
+    C = ctx.put(np.zeros((M + 1, N), cdt))
+    mxenc.gemm_i8(ctx, ctx.put(A), ctx.put(sa), M, K, K, slot, ctx.put(b), epi,
+                  ctx.put(R) if res else None, C, N)
+    got = C.host()
+    mxenc.check(L.mx_release_weight(ctx.handle, slot))
+    assert not got[M].any()
+    rows = np.unique(np.concatenate([np.arange(min(M, 130)), np.arange(max(0, M - 130), M)]))
+    Ar, sar = np.ascontiguousarray(A[rows]), np.ascontiguousarray(sa[rows])
+    c32 = np.zeros((rows.size, N), np.int32)
+    orc.orc_gemm_i8(P(Ar), rows.size, K, P(W), N, P(c32))
+    want = np.zeros((rows.size, N), np.float32)
+    orc.orc_dequantise_c(P(c32), rows.size, N, P(sar), P(ws), P(b), P(want))
+    if epi == POLY:
+        orc.orc_gelu_poly_inplace(P(want), want.size)
+    elif epi == ERF:
+        orc.orc_gelu_erf_inplace(P(want), want.size)
+    if res:
+        want += R[rows]
+    if cdt == np.uint16:
+        assert np.array_equal(got[rows], mxenc.to_bf16_bits(want))
+    elif epi == ERF:
+        # the device's erf and the host's differ by a few ulp: the bound of the
+        # exact-erf epilogue's own test against the host
+        assert np.max(np.abs(got[rows] - want)) < 1e-4
+    else:
+        assert np.array_equal(got[rows], want)
