@@ -171,33 +171,52 @@ __global__ __launch_bounds__(256) void layernorm_wave_k(
   const int lane = threadIdx.x & 63;
   const int64_t row = blockIdx.x * (int64_t)(blockDim.x / 64) + (threadIdx.x >> 6);
   if (row >= live_rows(rows, rows_dev)) return;
+  // gamma and beta, then every load of x, then every load of y, then the sums:
+  // a load behind the branch of the one before it would wait for its sum. What
+  // bounds this kernel over few rows is that chain of latencies: with it cut to
+  // one round of loads, and the butterflies off LDS, 19 rows of 384 take 2.6 us
+  // for 4.0 and 2,200 rows 4.4 for 5.3.
+  float2 gm[NP], bt[NP];
   float v[2 * NP];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const int64_t off = row * cols + i * 128 + lane * 2;
-    float a0, a1;
-    if (x_bf) {
-      const uint32_t p = *(const uint32_t *)((const uint16_t *)x + off);
-      a0 = bf2f(p & 0xFFFFu);
-      a1 = bf2f(p >> 16);
-    } else {
-      const float2 p = *(const float2 *)((const float *)x + off);
-      a0 = p.x;
-      a1 = p.y;
+    gm[i] = *(const float2 *)(gamma + i * 128 + lane * 2);
+    bt[i] = *(const float2 *)(beta + i * 128 + lane * 2);
+  }
+  const int64_t at = row * cols + lane * 2;
+  if (x_bf) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const uint32_t p = *(const uint32_t *)((const uint16_t *)x + at + i * 128);
+      v[2 * i] = bf2f(p & 0xFFFFu);
+      v[2 * i + 1] = bf2f(p >> 16);
     }
-    if (y) {
-      if (y_bf) {
-        const uint32_t p = *(const uint32_t *)((const uint16_t *)y + off);
-        a0 += bf2f(p & 0xFFFFu);
-        a1 += bf2f(p >> 16);
-      } else {
-        const float2 p = *(const float2 *)((const float *)y + off);
-        a0 += p.x;
-        a1 += p.y;
-      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const float2 p = *(const float2 *)((const float *)x + at + i * 128);
+      v[2 * i] = p.x;
+      v[2 * i + 1] = p.y;
     }
-    v[2 * i] = a0;
-    v[2 * i + 1] = a1;
+  }
+  if (y && y_bf) {
+    uint32_t w[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) w[i] = *(const uint32_t *)((const uint16_t *)y + at + i * 128);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      v[2 * i] += bf2f(w[i] & 0xFFFFu);
+      v[2 * i + 1] += bf2f(w[i] >> 16);
+    }
+  } else if (y) {
+    float2 w[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) w[i] = *(const float2 *)((const float *)y + at + i * 128);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      v[2 * i] += w[i].x;
+      v[2 * i + 1] += w[i].y;
+    }
   }
   float s = 0.0f;
 #pragma unroll
@@ -213,12 +232,9 @@ __global__ __launch_bounds__(256) void layernorm_wave_k(
   const float is = 1.0f / sqrtf(var + eps);
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const int c = i * 128 + lane * 2;
-    const float2 g = *(const float2 *)(gamma + c);
-    const float2 b = *(const float2 *)(beta + c);
-    const float r0 = __builtin_fmaf((v[2 * i] - mean) * is, g.x, b.x);
-    const float r1 = __builtin_fmaf((v[2 * i + 1] - mean) * is, g.y, b.y);
-    const int64_t off = row * cols + c;
+    const float r0 = __builtin_fmaf((v[2 * i] - mean) * is, gm[i].x, bt[i].x);
+    const float r1 = __builtin_fmaf((v[2 * i + 1] - mean) * is, gm[i].y, bt[i].y);
+    const int64_t off = at + i * 128;
     if (out_f32) *(float2 *)(out_f32 + off) = make_float2(r0, r1);
     if (out_bf16) *(uint32_t *)(out_bf16 + off) = pack_bf2(r0, r1);
   }
@@ -268,17 +284,31 @@ __global__ __launch_bounds__(256) void layernorm_wave4_k(
     gm[i] = *(const float4 *)(gamma + i * 256 + lane * 4);
     bt[i] = *(const float4 *)(beta + i * 256 + lane * 4);
   }
+  // Every load of x, then every load of y, then the sums (see above).
+  const int64_t at = row * cols + lane * 4;
   float4 v[NQ];
+  if (x_bf) {
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) {
-    const int64_t off = row * cols + i * 256 + lane * 4;
-    v[i] = ld4<ST>(x, x_bf, off);
-    if (y) {
-      const float4 w = ld4<ST>(y, y_bf, off);
-      v[i].x += w.x;
-      v[i].y += w.y;
-      v[i].z += w.z;
-      v[i].w += w.w;
+    for (int i = 0; i < NQ; ++i) v[i] = ld4<ST>(x, 1, at + i * 256);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) v[i] = ld4<ST>(x, 0, at + i * 256);
+  }
+  if (y) {
+    float4 w[NQ];
+    if (y_bf) {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) w[i] = ld4<ST>(y, 1, at + i * 256);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) w[i] = ld4<ST>(y, 0, at + i * 256);
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      v[i].x += w[i].x;
+      v[i].y += w[i].y;
+      v[i].z += w[i].z;
+      v[i].w += w[i].w;
     }
   }
   float s = 0.0f;

@@ -124,25 +124,38 @@ __global__ __launch_bounds__(256) void layernorm_quant_k(
       ia[i] = *(const float4 *)(ias + c);
     }
   }
+  // Every load of x, then every load of y, then the sums: a load behind the
+  // branch of the one before it would wait for its sum.
+  const int64_t at = row * cols + lane * 4;
   float4 v[NQ];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i)
+    v[i] = i * 256 + lane * 4 < cols ? load4<ST>(x, false, at + i * 256)
+                                     : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (y) {
+    float4 w[NQ];
+    if (y_bf) {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i)
+        w[i] = i * 256 + lane * 4 < cols ? load4<ST>(y, true, at + i * 256)
+                                         : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i)
+        w[i] = i * 256 + lane * 4 < cols ? load4<ST>(y, false, at + i * 256)
+                                         : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      v[i].x += w[i].x;
+      v[i].y += w[i].y;
+      v[i].z += w[i].z;
+      v[i].w += w[i].w;
+    }
+  }
   float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) {
-    const int c = i * 256 + lane * 4;
-    v[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (c < cols) {
-      const int64_t off = row * cols + c;
-      v[i] = load4<ST>(x, false, off);
-      if (y) {
-        const float4 w = load4<ST>(y, y_bf, off);
-        v[i].x += w.x;
-        v[i].y += w.y;
-        v[i].z += w.z;
-        v[i].w += w.w;
-      }
-    }
-    s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-  }
+  for (int i = 0; i < NQ; ++i) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
   const float mean = wave_sum(s) / (float)cols;
   float qs = 0.0f;
 #pragma unroll

@@ -91,16 +91,39 @@ __device__ __forceinline__ int64_t live_rows(int64_t rows, const int32_t *rows_d
   return r < 0 ? 0 : (r < rows ? r : rows);
 }
 
+// Wave-wide butterflies (xor 32, 16, 8, 4, 2, 1; every lane ends with the
+// result) on the vector ALU: v_permlane32_swap / v_permlane16_swap pair the
+// halves and the rows, and within a row of 16 a rotation by 8, 4, 2 and 1 reads
+// the xor partner's value (after the steps before it, lanes that far apart in
+// either direction hold the same one). The partner and the order are those of
+// __shfl_xor, so are the bits, without its six LDS round trips of ~100 cycles.
+// All 64 lanes must be active.
+template <int ROR>
+__device__ __forceinline__ float row_ror(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + ROR, 0xF, 0xF, true));
+}
+
+template <class Op>
+__device__ __forceinline__ float wave_butterfly(float v, Op op) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  v = op(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  v = op(v, row_ror<8>(v));
+  v = op(v, row_ror<4>(v));
+  v = op(v, row_ror<2>(v));
+  return op(v, row_ror<1>(v));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  return wave_butterfly(v, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
+  return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // gelu8 with the lane semantics of the reference's AVX2 branch
