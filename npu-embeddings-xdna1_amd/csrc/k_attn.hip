@@ -98,7 +98,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void attn_dma_k(const uint16_t *__res
                                                    int n_qblk, int force_logits,
                                                    const int32_t *__restrict__ seq_start,
                                                    const int32_t *__restrict__ order,
-                                                   int q_lim) {
+                                                   int q_lim, int rank_b) {
   constexpr int NKK = HD / 16, NHT = HD / 32;
   constexpr int ROWB = HD * 2, TILE = BKV * ROWB;  // bytes per row and per operand tile
   constexpr int SLOT = 2 * TILE + BKV * 4;         // K, V, mask row
@@ -117,6 +117,20 @@ __global__ __launch_bounds__(NW * 64, WPS) void attn_dma_k(const uint16_t *__res
     const int t = blk / H;
     qb = t % n_qblk;
     b = order[t / n_qblk];
+  } else if (rank_b > 0) {
+    // No launch order given, kv_len of rank_b <= 64 sequences: each wave ranks
+    // them by decreasing kv_len (ties by index), lane l holding sequence l's.
+    h = blk % H;
+    const int t = blk / H;
+    qb = t % n_qblk;
+    const int l = threadIdx.x & 63;
+    const int mine = kv_len[l < rank_b ? l : 0];
+    int rank = 0;
+    for (int o = 0; o < rank_b; ++o) {
+      const int other = __builtin_amdgcn_readlane(mine, o);
+      rank += other > mine || (other == mine && o < l) ? 1 : 0;
+    }
+    b = __builtin_ctzll(__ballot(l < rank_b && rank == t / n_qblk));
   } else {
     qb = blk % n_qblk;
     const int bh = blk / n_qblk;
@@ -417,16 +431,21 @@ hipError_t attention(const AttnArgs &a, hipStream_t s) {
   const int64_t blocks = a.B * a.H * n_qblk;
   const float sl2e = a.scale * 1.4426950408889634f;
   const int force_logits = a.scale > 0.0f ? 0 : 1;  // raw-score max needs scale > 0
+  // Sequences of uneven length without a launch order: the kernel ranks up to
+  // 64 of them itself (one per lane), so that the long ones' blocks start first
+  // and no CU is left with several of them at the end: 17 sequences of up to 433
+  // rows, 12 heads of 64, 21.6 -> 18.5 us. (The packed passes give the order.)
+  const int rank_b = !a.order && a.kv_len && a.B > 1 && a.B <= 64 ? (int)a.B : 0;
   // head_dim 64: 32-key tiles, a 4-slot ring, four blocks per CU; head_dim 32:
   // 64-key tiles, 3 slots, three blocks per CU.
   if (a.hd == 64)
     attn_dma_k<64, nw, 32, 4, 4><<<(unsigned)blocks, 64 * nw, 0, s>>>(
         a.qkv, a.ld_qkv, (int)a.S, (int)a.H, sl2e, a.add_mask, a.kv_len, a.ctx, a.ld_ctx,
-        n_qblk, force_logits, a.seq_start, a.order, (int)qs);
+        n_qblk, force_logits, a.seq_start, a.order, (int)qs, rank_b);
   else if (a.hd == 32)
     attn_dma_k<32, nw, 64, 3, 3><<<(unsigned)blocks, 64 * nw, 0, s>>>(
         a.qkv, a.ld_qkv, (int)a.S, (int)a.H, sl2e, a.add_mask, a.kv_len, a.ctx, a.ld_ctx,
-        n_qblk, force_logits, a.seq_start, a.order, (int)qs);
+        n_qblk, force_logits, a.seq_start, a.order, (int)qs, rank_b);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

@@ -1,4 +1,4 @@
-"""The GEMM's 16 x 16 MFMA forms and its paired 128 x 128 tile, at the sizes
+"""Small launches: the GEMM's 16 x 16 MFMA forms and its paired 128 x 128 tile, at the sizes
 where a tile, a slab ring or a wave's share of either can go wrong.
 
 Every tile runs the same chain of products over K for each element of C, so a
@@ -147,3 +147,30 @@ def test_small_tiles_i8(ctx, orc, M, K, N, epi, cdt, res, plan):
         assert np.max(np.abs(got[rows] - want)) < 1e-4
     else:
         assert np.array_equal(got[rows], want)
+
+
+@pytest.mark.parametrize("B,S,hd,lens", [
+    (2, 70, 64, [1, 70]),
+    (5, 200, 32, [200, 200, 3, 64, 129]),   # ties
+    (64, 40, 64, None),                     # the most sequences a wave ranks
+    (65, 40, 64, None),                     # one more: index order
+])
+def test_attention_ranks_uneven_sequences(ctx, B, S, hd, lens):
+    """Attention over sequences of uneven length without a launch order: every
+    sequence is computed once, bit for bit as when it is alone."""
+    print("case", B, S, hd, lens, flush=True)
+    H = 2
+    d = H * hd
+    rng = np.random.default_rng(B)
+    lens = np.array(lens if lens else rng.integers(1, S + 1, B), np.int32)
+    qkv = to_bf16_bits((rng.standard_normal((B * S, 3 * d)) * 0.5).astype(np.float32))
+    mask = np.where(np.arange(S)[None, :] < lens[:, None], 0.0, -1e30).astype(np.float32)
+    out = ctx.put(np.zeros((B * S, d), np.uint16))
+    mxenc.attention(ctx, ctx.put(qkv), 3 * d, B, S, H, hd, 1.0, ctx.put(mask), ctx.put(lens), out,
+                    d)
+    got = out.host().reshape(B, S, d)
+    for b in range(B):
+        one = ctx.put(np.zeros((S, d), np.uint16))
+        mxenc.attention(ctx, ctx.put(qkv[b * S:(b + 1) * S]), 3 * d, 1, S, H, hd, 1.0,
+                        ctx.put(mask[b:b + 1]), ctx.put(lens[b:b + 1]), one, d)
+        assert np.array_equal(got[b], one.host()), b
