@@ -176,6 +176,7 @@ hipError_t gemm_lds_launch(const GemmArgs &a, int grid, hipStream_t s);
 hipError_t gemm_lds_deep_launch(const GemmArgs &a, int grid, hipStream_t s);
 hipError_t gemm_lds_128_deep_launch(const GemmArgs &a, int grid, hipStream_t s);
 hipError_t gemm_lds_nc_launch(const GemmArgs &a, int grid, hipStream_t s);
+hipError_t gemm_lds16_glu_launch(const GemmArgs &a, int grid, hipStream_t s);
 template <int BM, int BN, int WGM, int WGN, int NS, int RB>
 hipError_t gemm_lds16_launch(const GemmArgs &a, int grid, hipStream_t s);
 
@@ -192,7 +193,8 @@ enum GemmPath {
   PATH_LDS16_128x128,      // 8 waves, 128-byte slabs, one block per CU
   PATH_LDS16_64x64,        // 256-byte slabs, three slots, one block per CU
   PATH_LDS16_64x64_PAIR,   // 256-byte slabs, two slots, two blocks per CU
-  PATH_LDS16_64x64_RB128   // 128-byte slabs, four slots, two blocks per CU
+  PATH_LDS16_64x64_RB128,  // 128-byte slabs, four slots, two blocks per CU
+  PATH_LDS16_64x128_GLU    // the gated FFN, 256-byte slabs, three slots, one block per CU
 };
 
 // The 256 x 256 tile on 128-byte slabs: a bf16 C without a residual or an
@@ -275,10 +277,15 @@ GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
       best_t = t;
     }
   }
-  // A few tiles of the gated FFN: the 64-byte form keeps three slabs in flight
-  // ahead, not one, and a launch this small waits on every slab's load.
-  if (best == PATH_LDS_128x128_DEEP && glu && ((M + 127) / 128) * ((N + 127) / 128) * 8 <= cus)
-    return PATH_LDS_128x128;
+  if (glu && best == PATH_LDS_128x128_DEEP) {
+    // Few tiles of the gated FFN: 64 x 128 ones of 16 x 16 MFMAs while each has
+    // a CU (an even number of column blocks per wave, which 64 x 64 lacks).
+    if (K % 128 == 0 && K >= 384 && ((M + 63) / 64) * ((N + 127) / 128) <= cus)
+      return PATH_LDS16_64x128_GLU;
+    // The 64-byte form keeps three slabs in flight ahead, not one: a launch of
+    // a few tiles waits on every slab's load.
+    if (((M + 127) / 128) * ((N + 127) / 128) * 8 <= cus) return PATH_LDS_128x128;
+  }
   return best;
 }
 
@@ -390,6 +397,7 @@ const char *gemm_plan_name(int64_t M, int64_t N, int64_t K, bool c_bf16, bool re
     case PATH_LDS16_128x128: return "lds_128x128x64_w64x32_ns4_mfma16_persistent";
     case PATH_LDS16_64x64: return "lds_64x64x128_w32x32_ns3_mfma16_persistent";
     case PATH_LDS16_64x64_PAIR: return "lds_64x64x128_w32x32_ns2_mfma16_persistent";
+    case PATH_LDS16_64x128_GLU: return "lds_64x128x128_w32x64_ns3_mfma16_persistent";
     case PATH_LDS16_64x64_RB128: return "lds_64x64x64_w32x32_ns4_mfma16_persistent";
     default: return "staged_128x128x64_w64x64";
   }
@@ -412,6 +420,7 @@ hipError_t gemm(const GemmArgs &a, hipStream_t s) {
     case PATH_LDS_128x128_DEEP: return gemm_lds_128_deep_launch(a, 2 * cu_count(), s);
     case PATH_LDS16_128x128: return gemm_lds16_launch<128, 128, 2, 4, 4, 128>(a, cu_count(), s);
     case PATH_LDS16_64x64: return gemm_lds16_launch<64, 64, 2, 2, 3, 256>(a, cu_count(), s);
+    case PATH_LDS16_64x128_GLU: return gemm_lds16_glu_launch(a, cu_count(), s);
     case PATH_LDS16_64x64_PAIR:
       return gemm_lds16_launch<64, 64, 2, 2, 2, 256>(a, 2 * cu_count(), s);
     case PATH_LDS16_64x64_RB128:

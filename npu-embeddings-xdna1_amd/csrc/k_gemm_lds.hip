@@ -144,7 +144,17 @@ hipError_t gemm_lds_128_deep_launch(const GemmArgs &a, int grid, hipStream_t s) 
   }
 }
 
-// The 16 x 16 MFMA forms (gemm_path() says which product takes which), one
+// The gated FFN on 16 x 16 MFMAs: a few tiles, one per CU.
+hipError_t gemm_lds16_glu_launch(const GemmArgs &a, int grid, hipStream_t s) {
+  if (!a.c_bf16 || a.residual) return hipErrorInvalidValue;
+  if (a.epilogue == EPI_GLU_SILU)
+    return gemm_lds_launch_t<64, 128, 2, 2, 3, EPI_GLU_SILU, false, true, 256, true>(a, grid, s);
+  if (a.epilogue == EPI_GLU_GELU)
+    return gemm_lds_launch_t<64, 128, 2, 2, 3, EPI_GLU_GELU, false, true, 256, true>(a, grid, s);
+  return hipErrorInvalidValue;
+}
+
+// The 16 x 16 MFMA forms (pick_deep() says which product takes which), one
 // tile configuration, an activation and an optional fp32 residual.
 template <int BM, int BN, int WGM, int WGN, int NS, int RB>
 hipError_t gemm_lds16_launch(const GemmArgs &a, int grid, hipStream_t s) {

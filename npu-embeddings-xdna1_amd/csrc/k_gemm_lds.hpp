@@ -272,7 +272,6 @@ __device__ __forceinline__ void gemm_lds_body(
   typedef typename PT::frag frag_t;
   typedef typename PT::acc acc_t;
   typedef typename PT::acc4 acc4_t;
-  static_assert(!M16 || EPI < 8 || (EPI & EPI_NARROW_C), "16 x 16 tiles: not the gated FFN");
   static_assert(I8 || !RAW, "RAW is the int8 datapath's");
   static_assert(!RAW || (EPI == 0 && !RES && !CBF), "RAW stores the accumulators as they are");
   constexpr int TM = Cfg::TM, TN = Cfg::TN, ESZ = Cfg::ESZ;
@@ -612,34 +611,76 @@ __device__ __forceinline__ void gemm_lds_body(
         // Columns 16u + e (lo) and 16u + 8 + e (hi) of accumulator block
         // 2j + jj give C's column 8(2jj + u) + e: each pair rounds to bf16 as
         // the unfused GEMM's C does, then lo * act(hi) rounds once more.
-        const float sa = I8 ? sal[wm * Cfg::WM + i * 32 + li] : 0.0f;
+        if constexpr (M16) {
+          // Column 16u + e (lo, e < 8) sits in lanes 0 .. 31 and 16u + 8 + e
+          // (hi) 32 lanes on, of tile u. One v_permlane32_swap of the two
+          // tiles' pairs gives lanes 0 .. 31 both halves of tile 0's columns
+          // and lanes 32 .. 63 both of tile 1's: C's columns 4 (lane / 16) ..
+          // + 3 of the block's 16, the place of tile jj in the staged block.
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          const int ja = 2 * j + jj;
-          const int cl = wn * Cfg::WN + ja * 32;
+          for (int jj = 0; jj < 2; ++jj) {
+            const int ja = 2 * j + jj;
+            const int cl = wn * Cfg::WN + ja * 32;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            b[q] = has_bias ? *(const float4 *)(bl + cl + cq(q))
-                            : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (I8) w[q] = *(const float4 *)(wsl + cl + cq(q));
-          }
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const float bl4[4] = {b[2 * u].x, b[2 * u].y, b[2 * u].z, b[2 * u].w};
-            const float bh4[4] = {b[2 * u + 1].x, b[2 * u + 1].y, b[2 * u + 1].z,
-                                  b[2 * u + 1].w};
-            const float wl4[4] = {w[2 * u].x, w[2 * u].y, w[2 * u].z, w[2 * u].w};
-            const float wh4[4] = {w[2 * u + 1].x, w[2 * u + 1].y, w[2 * u + 1].z,
-                                  w[2 * u + 1].w};
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const uint32_t h = pack_bf2_hw(pre(ja, i, 2 * u, e, bl4[e], wl4[e], sa),
-                                             pre(ja, i, 2 * u + 1, e, bh4[e], wh4[e], sa));
-              o[e] = bf2f(h & 0xFFFFu) * glu_act<GACT>(bf2f(h >> 16));
+            for (int q = 0; q < 4; ++q) {
+              b[q] = has_bias ? *(const float4 *)(bl + cl + cq(q))
+                              : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+              if (I8) w[q] = *(const float4 *)(wsl + cl + cq(q));
             }
-            pk[2 * (2 * jj + u)] = pack_bf2(o[0], o[1]);
-            pk[2 * (2 * jj + u) + 1] = pack_bf2(o[2], o[3]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {  // row half
+              const float sa = I8 ? sal[wm * Cfg::WM + i * 32 + rq(2 * u)] : 0.0f;
+              uint32_t t[2][2];
+#pragma unroll
+              for (int x = 0; x < 2; ++x) {
+                const int q = 2 * u + x;
+                const float bb[4] = {b[q].x, b[q].y, b[q].z, b[q].w};
+                const float ww[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                  t[x][h] = pack_bf2_hw(pre(ja, i, q, 2 * h, bb[2 * h], ww[2 * h], sa),
+                                        pre(ja, i, q, 2 * h + 1, bb[2 * h + 1], ww[2 * h + 1], sa));
+              }
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const auto r = __builtin_amdgcn_permlane32_swap(t[0][h], t[1][h], false, false);
+                const uint32_t lo = r[0], hi = r[1];
+                pk[2 * (2 * u + jj) + h] =
+                    pack_bf2(bf2f(lo & 0xFFFFu) * glu_act<GACT>(bf2f(hi & 0xFFFFu)),
+                             bf2f(lo >> 16) * glu_act<GACT>(bf2f(hi >> 16)));
+              }
+            }
+          }
+        } else {
+          const float sa = I8 ? sal[wm * Cfg::WM + i * 32 + li] : 0.0f;
+#pragma unroll
+          for (int jj = 0; jj < 2; ++jj) {
+            const int ja = 2 * j + jj;
+            const int cl = wn * Cfg::WN + ja * 32;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              b[q] = has_bias ? *(const float4 *)(bl + cl + cq(q))
+                              : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+              if (I8) w[q] = *(const float4 *)(wsl + cl + cq(q));
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const float bl4[4] = {b[2 * u].x, b[2 * u].y, b[2 * u].z, b[2 * u].w};
+              const float bh4[4] = {b[2 * u + 1].x, b[2 * u + 1].y, b[2 * u + 1].z,
+                                    b[2 * u + 1].w};
+              const float wl4[4] = {w[2 * u].x, w[2 * u].y, w[2 * u].z, w[2 * u].w};
+              const float wh4[4] = {w[2 * u + 1].x, w[2 * u + 1].y, w[2 * u + 1].z,
+                                    w[2 * u + 1].w};
+              float o[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const uint32_t h = pack_bf2_hw(pre(ja, i, 2 * u, e, bl4[e], wl4[e], sa),
+                                               pre(ja, i, 2 * u + 1, e, bh4[e], wh4[e], sa));
+                o[e] = bf2f(h & 0xFFFFu) * glu_act<GACT>(bf2f(h >> 16));
+              }
+              pk[2 * (2 * jj + u)] = pack_bf2(o[0], o[1]);
+              pk[2 * (2 * jj + u) + 1] = pack_bf2(o[2], o[3]);
+            }
           }
         }
       } else {

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import mxenc
-from mxenc import from_bf16_bits, to_bf16_bits
+from mxenc import from_bf16_bits, synth, to_bf16_bits
 from orc import P
 
 pytestmark = pytest.mark.gpu
@@ -147,6 +147,29 @@ def test_small_tiles_i8(ctx, orc, M, K, N, epi, cdt, res, plan):
         assert np.max(np.abs(got[rows] - want)) < 1e-4
     else:
         assert np.array_equal(got[rows], want)
+
+
+@pytest.mark.parametrize("name,B,S", [("nomic", 1, 1), ("gte", 1, 65), ("nomic", 3, 131)])
+def test_small_gated_ffn(ctx, name, B, S):
+    """The fused gated FFN on 64 x 128 tiles: bit for bit the GEMM and the
+    gated-FFN pass apart."""
+    print("case", name, B, S, flush=True)
+    m = synth.make_model(name, layers=2, ln_random=True)
+    enc = mxenc.Encoder(ctx, m)
+    x = np.random.default_rng(B * S).standard_normal((B * S, m["hidden"])).astype(np.float32)
+
+    def run(fused):
+        enc.set_fusion(fused)
+        dx = ctx.put(x)
+        enc.run(dx, None, None, B, S)
+        return dx.host()
+
+    try:
+        a, b = run(True), run(False)
+        assert np.isfinite(a).all()
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    finally:
+        enc.close()
 
 
 @pytest.mark.parametrize("B,S,hd,lens", [
