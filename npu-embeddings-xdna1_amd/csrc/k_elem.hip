@@ -740,7 +740,8 @@ constexpr int64_t ORDER_MAX_B = 8192;
 __global__ __launch_bounds__(256) void pack_plan_k(const int32_t *__restrict__ kv_len, int64_t B,
                                                    int32_t *__restrict__ seq_start,
                                                    int32_t *__restrict__ order,
-                                                   int32_t *__restrict__ total_out) {
+                                                   int32_t *__restrict__ total_out,
+                                                   uint64_t *note, uint64_t bound) {
   if (threadIdx.x == 0) {
     int32_t acc = 0;
     for (int64_t b = 0; b < B; ++b) {
@@ -749,6 +750,9 @@ __global__ __launch_bounds__(256) void pack_plan_k(const int32_t *__restrict__ k
     }
     seq_start[B] = acc;
     if (total_out) *total_out = acc;
+    if (note)
+      __hip_atomic_store(note, bound << 32 | (uint64_t)(uint32_t)acc, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
   }
   if (!order) return;
   for (int64_t b = threadIdx.x; b < B; b += blockDim.x) {
@@ -1141,8 +1145,9 @@ hipError_t gather_cls(const float *x, const uint16_t *ctx, const int32_t *seq_st
 }
 
 hipError_t pack_plan(const int32_t *kv_len, int64_t B, int32_t *seq_start, int32_t *order,
-                     hipStream_t s, int32_t *total_out) {
-  pack_plan_k<<<1, 256, 0, s>>>(kv_len, B, seq_start, order, total_out);
+                     hipStream_t s, int32_t *total_out, uint64_t *note, int64_t bound) {
+  if (bound < 0 || bound > INT32_MAX) note = nullptr;
+  pack_plan_k<<<1, 256, 0, s>>>(kv_len, B, seq_start, order, total_out, note, (uint64_t)bound);
   return hipGetLastError();
 }
 

@@ -341,6 +341,13 @@ int mx_stream_create(mx_ctx *ctx, mx_stream **out) {
     delete s;
     return hip_fail(e, "stream refusal flag");
   }
+  // Only a hint rides on it: without pinned memory the stream goes on.
+  if (hipHostMalloc((void **)&s->note, sizeof(uint64_t), hipHostMallocDefault) == hipSuccess) {
+    *s->note = 0;
+  } else {
+    s->note = nullptr;
+    (void)hipGetLastError();
+  }
   *out = s;
   return MX_OK;
 }
@@ -350,6 +357,7 @@ void mx_stream_destroy(mx_stream *s) {
   if (use_device(s->ctx) == MX_OK) {
     (void)hipStreamSynchronize(s->stream);
     (void)hipFree(s->err_dev);
+    if (s->note) (void)hipHostFree(s->note);
     (void)hipStreamDestroy(s->stream);
   }
   delete s;

@@ -1349,8 +1349,8 @@ int pass_plan(mx_encoder *enc, Pass &p) {
   // the refusal flag at the end of the call: the next pass's tile hint.
   if (e == hipSuccess)
     e = mxk::pack_plan(p.w.kv_len, p.B, p.w.seq_start, p.w.seq_start + p.B + 1, p.s->stream,
-                       p.s->err_dev + 1);
-  if (e == hipSuccess) p.s->plan_bound = p.B * p.S;
+                       p.s->err_dev + 1, p.B > 1 ? p.s->note : nullptr, p.B * p.S);
+  if (e == hipSuccess) p.s->plan_bound = p.B > 1 ? p.B * p.S : 0;
   return e == hipSuccess ? MX_OK : hip_fail(e, "embed launch");
 }
 
@@ -1382,7 +1382,7 @@ int pass_rows(mx_encoder *enc, Pass &p, Carver *carve) {
           enc->packed_sq += L * L;
         }
       }
-    } else if (carve || p.s->last_rows <= 0) {
+    } else if (carve || (B > 1 && p.s->last_rows <= 0)) {
       // (also the first packed pass on a stream: no earlier total to pick the
       // GEMM tiles by)
       int32_t t = 0;
@@ -1390,9 +1390,9 @@ int pass_rows(mx_encoder *enc, Pass &p, Carver *carve) {
                          p.s->stream);
       if (e == hipSuccess) e = hipStreamSynchronize(p.s->stream);
       total = t;
-      if (e == hipSuccess) p.s->saw_rows(t, B * S);
+      if (e == hipSuccess) p.s->saw_rows(t, B > 1 ? B * S : 0);
     } else {
-      enc->live = mx::Live{p.w.seq_start + B, p.s->expected_rows(B * S)};
+      enc->live = mx::Live{p.w.seq_start + B, p.s->expected_rows(B, S)};
       enc->live_bound = B * S;
     }
     if (e != hipSuccess) return hip_fail(e, "reading the packed row count");

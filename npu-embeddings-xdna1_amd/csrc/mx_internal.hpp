@@ -81,15 +81,27 @@ struct mx_stream {
   // for. (The bare count misjudges a pass of another size: batches of 64 x 512
   // queued behind a query of three passages ran on the query's tiles, 6.1 ms a
   // bge-base batch against 5.0.)
+  // A single sequence fills its own width and says nothing of a batch: it
+  // leaves the share as it was.
   int last_rows = 0;
   int64_t last_bound = 0;
-  int64_t plan_bound = 0;  // B * S of the last pass queued
+  int64_t plan_bound = 0;  // B * S of the last pass queued, 0 for one sequence
+  // The same pair as the last completed pass's plan wrote it (bound << 32 |
+  // rows, one 8-byte store into pinned host memory; 0 before the first), for
+  // passes queued without a wait between them. Null: pinned memory refused.
+  uint64_t *note = nullptr;
   void saw_rows(int rows, int64_t bound) {
     if (rows <= 0 || bound <= 0) return;
     last_rows = rows;
     last_bound = bound;
   }
-  int64_t expected_rows(int64_t bound) const {
+  int64_t expected_rows(int64_t B, int64_t S) {
+    const int64_t bound = B * S;
+    if (note) {
+      const uint64_t v = __atomic_load_n(note, __ATOMIC_RELAXED);
+      saw_rows((int)(uint32_t)v, (int64_t)(v >> 32));
+    }
+    if (B == 1 || last_bound <= 0) return bound;
     const double r = (double)last_rows / (double)last_bound * (double)bound;
     return r < 1.0 ? 1 : r < (double)bound ? (int64_t)r : bound;
   }

@@ -46,9 +46,11 @@ hipError_t gather_cls(const float *x, const uint16_t *ctx, const int32_t *seq_st
 // packed rows) and, when order is non-null, order[0..B) = the sequence
 // indices by decreasing kv_len (attention's launch order); the embedding sum
 // of the rows s < kv_len[b] into packed row seq_start[b] + s, with
-// row_pos[packed row] = s. total_out (nullable): a second copy of seq_start[B].
+// row_pos[packed row] = s. total_out (nullable): a second copy of seq_start[B];
+// note (nullable, host memory the device can write): bound << 32 | seq_start[B].
 hipError_t pack_plan(const int32_t *kv_len, int64_t B, int32_t *seq_start, int32_t *order,
-                     hipStream_t s, int32_t *total_out = nullptr);
+                     hipStream_t s, int32_t *total_out = nullptr, uint64_t *note = nullptr,
+                     int64_t bound = 0);
 hipError_t embed_sum_packed(const int32_t *ids, int64_t B, int64_t S, int64_t d,
                             const float *word, int64_t vocab, const float *pos,
                             const float *type0, const int32_t *kv_len, const int32_t *seq_start,
