@@ -80,7 +80,7 @@ struct mx_stream {
   // packed pass on this stream takes the row count its GEMM tiles are chosen
   // for. (The bare count misjudges a pass of another size: batches of 64 x 512
   // queued behind a query of three passages ran on the query's tiles, 6.1 ms a
-  // bge-base batch against 5.0.)
+  // bge-base batch against 4.1.)
   // A single sequence fills its own width and says nothing of a batch: it
   // leaves the share as it was.
   int last_rows = 0;
