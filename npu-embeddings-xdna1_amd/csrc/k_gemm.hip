@@ -301,7 +301,7 @@ GemmPath pick(const GemmArgs &a) {
       a.N % 64 == 0 &&
       ((a.M + 63) / 64) * (a.N / 64) <= cu_count())
     return PATH_LDS16_64x64;
-  int t = gemm_lds_tile(m, a.N, false);
+  int t = gemm_lds_tile(m, a.N);
   if (t == 1 && glu) t = 0;  // 96-column waves cannot pair blocks
   return paths[t];
 }
@@ -312,16 +312,16 @@ GemmPath pick(const GemmArgs &a) {
 // last round costs a whole one) times the tile's area over its relative
 // throughput per unit area, measured on MI355X on the encoder's GEMM shapes
 // when every tile count is a whole number of rounds (256 x 256: 1.0, 256 x
-// 192: 0.88, 128 x 256: 0.86, 128 x 128: 0.65; the 256 x 256 tile on
-// 128-byte slabs: 1.1). The 256 x 192 tile wins where N = 768 leaves 256 x
+// 192: 0.88, 128 x 256: 0.86, 128 x 128: 0.65), for the products that have
+// 64-byte slabs only. The 256 x 192 tile wins where N = 768 leaves 256 x
 // 256 tiles at 1.5 rounds; small problems take the small tiles that spread
 // over the most CUs.
-int gemm_lds_tile(int64_t M, int64_t N, bool deep) {
+int gemm_lds_tile(int64_t M, int64_t N) {
   struct Cand {
     int bm, bn;
     double eff;
   };
-  const Cand cands[] = {{256, 256, deep ? 1.1 : 1.0}, {256, 192, 0.88}, {128, 256, 0.86},
+  const Cand cands[] = {{256, 256, 1.0}, {256, 192, 0.88}, {128, 256, 0.86},
                         {128, 128, 0.65}};
   const int64_t G = cu_count();
   int best = 3;

@@ -141,7 +141,7 @@ hipError_t launch_nc(const mxk::GemmI8Args &a, int grid, hipStream_t s) {
                             : launch_t<BM, BN, WGM, WGN, NS, NC | 2, false, 0>(a, grid, s);   \
     default: return hipErrorInvalidValue;                                                     \
   }
-  if (mxk::gemm_lds_tile(mxk::gemm_pick_rows(a.M, a.m_hint), a.N, false) == 0) {
+  if (mxk::gemm_lds_tile(mxk::gemm_pick_rows(a.M, a.m_hint), a.N) == 0) {
     MX_I8_NC(256, 256, 2, 4, 3)
   }
   MX_I8_NC(128, 128, 2, 2, 4)

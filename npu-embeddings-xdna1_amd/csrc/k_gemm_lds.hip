@@ -198,7 +198,7 @@ hipError_t gemm_lds_nc_launch(const GemmArgs &a, int grid, hipStream_t s) {
   }                                                                                       \
   if (e == 0) return gemm_lds_launch_t<BM, BN, WGM, WGN, NS, NC, false, false>(a, grid, s); \
   return hipErrorInvalidValue;
-  if (gemm_lds_tile(gemm_pick_rows(a.M, a.m_hint), a.N, false) == 0) {
+  if (gemm_lds_tile(gemm_pick_rows(a.M, a.m_hint), a.N) == 0) {
     MX_LDS_NC(256, 256, 2, 4, 3)
   }
   MX_LDS_NC(128, 128, 2, 2, 4)

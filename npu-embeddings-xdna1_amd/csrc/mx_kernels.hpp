@@ -103,9 +103,9 @@ hipError_t glu_interleave(const void *src, void *dst, int64_t f, int64_t row_byt
                           hipStream_t s);
 
 // The LDS-pipelined kernel's tile for an M x N product (0: 256x256, 1: 256x192,
-// 2: 128x256, 3: 128x128; deep: the 256 x 256 tile would run on 128-byte
-// slabs) and the resident blocks of a persistent launch.
-int gemm_lds_tile(int64_t M, int64_t N, bool deep);
+// 2: 128x256, 3: 128x128) on 64-byte slabs, and the resident blocks of a
+// persistent launch.
+int gemm_lds_tile(int64_t M, int64_t N);
 // The row count a launch's tile is chosen for: the hint when one is given
 // (and below M), else M.
 inline int64_t gemm_pick_rows(int64_t M, int64_t hint) { return hint > 0 && hint < M ? hint : M; }
