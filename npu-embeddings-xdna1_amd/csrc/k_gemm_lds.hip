@@ -20,9 +20,13 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_lds_k(
       rows_dev);
 }
 
-// The body's 16 x 16 MFMA form.
+// The body's 16 x 16 MFMA form. Two waves per SIMD, or one (all 512 registers)
+// for a 64-column wave on 256-byte slabs: its two whole-slab sets and the
+// accumulators need some 340, and its ring leaves a CU one block of four waves.
+// Held to 256, it kept 146 of them in scratch: the gated FFN-up of 20 rows
+// (K 768, N 6144) took 22.4 us, 8.2 so.
 template <int BM, int BN, int WGM, int WGN, int NS, int EPI, bool RES, bool CBF, int RB>
-__global__ __launch_bounds__(WGM *WGN * 64, 2) void gemm_lds16_k(
+__global__ __launch_bounds__(WGM *WGN * 64, RB == 256 && BN / WGN > 32 ? 1 : 2) void gemm_lds16_k(
     const uint16_t *__restrict__ A, int64_t lda, const uint16_t *__restrict__ Wt, int M, int N,
     int K, const float *__restrict__ bias, const float *residual, void *C, int64_t ldc,
     int tiles_m, int tiles_n, const int32_t *rows_dev) {
