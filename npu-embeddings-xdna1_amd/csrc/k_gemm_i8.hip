@@ -38,9 +38,13 @@ template <int BM, int BN, int WGM, int WGN, int NS, int EPI, bool RES, int OUT, 
           bool M16 = false>
 hipError_t launch_t(const mxk::GemmI8Args &a, int grid, hipStream_t s) {
   using Cfg = LdsCfg<BM, BN, WGM, WGN, NS, true, stg_kind(OUT == 1, RES), RB>;
-  auto kern = gemm_i8_k<BM, BN, WGM, WGN, NS, EPI, RES, OUT, RB>;
-  if constexpr (M16) kern = gemm_i8_16_k<BM, BN, WGM, WGN, NS, EPI, RES, OUT, RB>;
-  static bool attr_set = false;
+  constexpr auto kern = [] {
+    if constexpr (M16)
+      return gemm_i8_16_k<BM, BN, WGM, WGN, NS, EPI, RES, OUT, RB>;
+    else
+      return gemm_i8_k<BM, BN, WGM, WGN, NS, EPI, RES, OUT, RB>;
+  }();
+   static bool attr_set = false;
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(
         (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);

@@ -44,9 +44,13 @@ template <int BM, int BN, int WGM, int WGN, int NS, int EPI, bool RES, bool CBF,
           bool M16 = false>
 hipError_t gemm_lds_launch_t(const GemmArgs &a, int grid, hipStream_t s) {
   using Cfg = LdsCfg<BM, BN, WGM, WGN, NS, false, stg_kind(CBF, RES), RB>;
-  auto kern = gemm_lds_k<BM, BN, WGM, WGN, NS, EPI, RES, CBF, RB>;
-  if constexpr (M16) kern = gemm_lds16_k<BM, BN, WGM, WGN, NS, EPI, RES, CBF, RB>;
-  static bool attr_set = false;
+  constexpr auto kern = [] {
+    if constexpr (M16)
+      return gemm_lds16_k<BM, BN, WGM, WGN, NS, EPI, RES, CBF, RB>;
+    else
+      return gemm_lds_k<BM, BN, WGM, WGN, NS, EPI, RES, CBF, RB>;
+  }();
+   static bool attr_set = false;
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(
         (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);

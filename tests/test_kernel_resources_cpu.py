@@ -60,3 +60,12 @@ def test_gemm_kernels_use_no_scratch(kernels):
     assert len(gemm) > 100
     # 8 bytes: one register of an epilogue, out of the main loop
     assert not {n: s for n, s in gemm.items() if s > 8}
+
+
+def test_one_mfma_form_per_tile(kernels):
+    """A tile's kernel exists in the MFMA form that its launcher takes, not in
+    the other as well."""
+    args = lambda name: {n[len(name):] for n in kernels if n.startswith(name + "<")}  # noqa: E731
+    for a, b in (("gemm_lds_k", "gemm_lds16_k"), ("gemm_i8_k", "gemm_i8_16_k")):
+        assert len(args(a)) > 20 and len(args(b)) > 5
+        assert not args(a) & args(b)
