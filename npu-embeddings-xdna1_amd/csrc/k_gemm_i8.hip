@@ -44,7 +44,7 @@ hipError_t launch_t(const mxk::GemmI8Args &a, int grid, hipStream_t s) {
     else
       return gemm_i8_k<BM, BN, WGM, WGN, NS, EPI, RES, OUT, RB>;
   }();
-   static bool attr_set = false;
+  static bool attr_set = false;
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(
         (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);

@@ -50,7 +50,7 @@ hipError_t gemm_lds_launch_t(const GemmArgs &a, int grid, hipStream_t s) {
     else
       return gemm_lds_k<BM, BN, WGM, WGN, NS, EPI, RES, CBF, RB>;
   }();
-   static bool attr_set = false;
+  static bool attr_set = false;
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(
         (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
