@@ -843,9 +843,15 @@ __device__ __forceinline__ void gemm_lds_body(
         // the writes of 16 rows and the reads of 4 rows x 4 chunks each cover
         // all 64 banks once. Everything else stages fp32 rows (the residual is
         // added before the one rounding).
+        // A row's a_scale is read before the staging writes, not again behind
+        // each (rq(q) is rq(0) or rq(2)).
+        float sas[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          sas[u] = I8 && !RAW ? sal[wm * Cfg::WM + i * 32 + rq(2 * u)] : 0.0f;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const float sa = I8 && !RAW ? sal[wm * Cfg::WM + i * 32 + rq(q)] : 0.0f;
+          const float sa = sas[q >> 1];
           float4 v;
           if (RAW) {
             v.x = __int_as_float((int)acc_at(j, i, q * 4 + 0));
