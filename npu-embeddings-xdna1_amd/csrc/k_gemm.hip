@@ -216,16 +216,19 @@ bool lds_path_ok(const GemmArgs &a) {
 // CU, one after another or (two blocks per CU) in pairs, so
 //   us = start + K * (pair * (n / 2) + one * (n % 2)) + n * tile
 //        (+ n * res: an fp32 C with a residual),
-// `one` and `pair` the cost per K of one tile on a CU and of two. Fitted to 220
-// products on an MI355X (M 100 to 9000, K and N 384 to 5120, weights rotating
-// over eight copies; 8-9 % rms per path). Against the tile areas alone, by which these
-// products took a tile before, the choice takes 0.73 of the time in the
-// geometric mean over them: 700 x 1024 x 4096 40.7 -> 16.3 us (K = 4096),
-// 1500 x 768 x 768 11.1 -> 7.9, 3000 x 1280 x 5120 with a residual 55 -> 51.
-// The worst product loses 4 % (6000 x 384 x 384, 7.2 -> 7.5 us). The bounds on
-// K keep a tile at least as deep as the ring: a ring that held slabs of three
-// tiles would hold two tiles' epilogue vectors in one place. 64-column tiles
-// take whole column tiles only (every layer of a model has them).
+// `one` and `pair` the cost per K of one tile on a CU and of two: constants
+// fitted to products measured on an MI355X (weights rotating over eight copies),
+// but for the 128 x 256 row's cost per K, the best of four tried, and the 256 x
+// 256 row's cost per tile, raised from 3.28 for the sake of K below 512. Over
+// 700 further products (M 1 to 40,000, N 64 to 6144, K 128 to 5120; bf16, fp32 +
+// residual, gated) the choice takes 0.66 of the time of the choice by tile areas
+// over the 32 x 32 MFMA tiles alone, in the geometric mean, and the best tile of
+// each 0.66 too (1.009 between the two); the longest loses 3 % by it (38,303 x
+// 1000 x 1536, 111.9 -> 115.4 us). 700 x 1024 x 4096 takes 16.5 us for 42.2, 1500
+// x 768 x 768 7.9 for 11.1, 3000 x 1280 x 5120 with a residual 49.3 for 54.4, 300
+// x 768 x 128 4.55 for 4.88. The bounds on K keep a tile at least as deep as the
+// ring: a ring that held slabs of three tiles would hold two tiles' epilogue
+// vectors in one place. A 64-column tile over a ragged N is left out unmeasured.
 GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
   struct Cost {
     GemmPath path;
@@ -233,7 +236,7 @@ GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
     double start, one, pair, tile, res;
   };
   static const Cost costs[] = {
-      {PATH_LDS_256x256_DEEP, 256, 256, 3.27, .0198, .0396, 3.28, 3.84},
+      {PATH_LDS_256x256_DEEP, 256, 256, 3.27, .0198, .0396, 4.00, 3.84},
       {PATH_LDS_256x192, 256, 192, 1.73, .0183, .0366, 4.54, 2.54},
       {PATH_LDS_128x256, 128, 256, 0.00, .0150, .0300, 5.11, 1.73},
       {PATH_LDS_128x128_DEEP, 128, 128, 0.63, .0103, .0135, 2.55, 2.64},
@@ -246,30 +249,30 @@ GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
   double best_t = 0.0;
   for (const Cost &c : costs) {
     const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const int64_t n = (tiles + cus - 1) / cus;
+    // The gated FFN needs an even number of column blocks per wave. More than
+    // three 64 x 64 tiles to a CU read W too often for the cost per K: 1065 x 3840
+    // x 3072 with a residual takes 60 us on four, 47 on the 128 x 128 pairs.
+    const bool small = !glu && N % 64 == 0 && n <= 3;
     switch (c.path) {
       case PATH_LDS_256x192:  // 96-column waves cannot pair the gated FFN's blocks
         if (glu) continue;
-        break;
-      case PATH_LDS_128x128_DEEP:
-        // Below K = 512 the pairs' gain on the 128 x 256 tile is 1 us in 12.
-        if (K < 512 && !glu) continue;
         break;
       case PATH_LDS16_128x128:
         if (glu || K < 256) continue;
         break;
       case PATH_LDS16_64x64:
-        if (K % 128 || K < 384 || glu || N % 64) continue;
+        if (!small || K % 128 || K < 384) continue;
         break;
       case PATH_LDS16_64x64_PAIR:
-        if (K % 128 || K < 256 || glu || N % 64) continue;
+        if (!small || K % 128 || K < 256) continue;
         break;
       case PATH_LDS16_64x64_RB128:
         // Only where K has no 256-byte slabs: they halve the barriers per K.
-        if (K % 128 == 0 || K < 256 || glu || N % 64) continue;
+        if (!small || K % 128 == 0 || K < 256) continue;
         break;
       default: break;
     }
-    const int64_t n = (tiles + cus - 1) / cus;
     const double t = c.start + (double)K * (c.pair * (double)(n / 2) + c.one * (double)(n % 2)) +
                      (double)n * (c.tile + (res ? c.res : 0.0));
     if (best_t == 0.0 || t < best_t) {

@@ -1017,9 +1017,9 @@ __device__ __forceinline__ void gemm_lds_body(
     } else {
       wait_slab<Cfg::LOADS_LO, NS - 2, EPI_STORES>(ahead, stores_young);
     }
-    // (max and a subtraction, both scalar: a decrement behind a test of the same
-    // count went through a vector register and back on every slab: 10 to 12
-    // cycles in a chain that a lone tile waits out, 27.5 us for 26.3 at 80 slabs)
+    // (max and a subtraction, both scalar: the same decrement behind a test went
+    // through a vector register and back on every slab, 15 ns of a lone tile's
+    // chain)
     epi_left = max(epi_left, 1) - 1;
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
