@@ -117,32 +117,50 @@ __global__ __launch_bounds__(NW * 64, WPS) void attn_dma_k(const uint16_t *__res
     const int t = blk / H;
     qb = t % n_qblk;
     b = order[t / n_qblk];
-  } else if (rank_b > 0) {
-    // No launch order given, kv_len of rank_b <= 64 sequences: each wave ranks
-    // them by decreasing kv_len (ties by index), lane l holding sequence l's.
-    h = blk % H;
-    const int t = blk / H;
-    qb = t % n_qblk;
-    const int l = threadIdx.x & 63;
-    const int mine = kv_len[l < rank_b ? l : 0];
-    int rank = 0;
-    for (int o = 0; o < rank_b; ++o) {
-      const int other = __builtin_amdgcn_readlane(mine, o);
-      rank += other > mine || (other == mine && o < l) ? 1 : 0;
-    }
-    b = __builtin_ctzll(__ballot(l < rank_b && rank == t / n_qblk));
   } else {
     qb = blk % n_qblk;
     const int bh = blk / n_qblk;
     h = bh % H;
     b = bh / H;
   }
+  int kvl = -1;
+  if (rank_b > 0) {
+    // No launch order given, kv_len of rank_b <= 64 sequences, lane l holding
+    // sequence l's. All of one length: the block order above. Else the order of
+    // the packed passes (every head of a query block, then the next), over the
+    // sequences by decreasing kv_len (ties by index): the one of rank k is
+    // selected bit by bit from the top, the lanes left in m either having the
+    // bit (k counts among them) or losing those that have it.
+    const int l = threadIdx.x & 63;
+    int len = kv_len[l < rank_b ? l : 0];
+    len = len < 1 ? 1 : (len > S ? S : len);
+    if (__ballot(len != __builtin_amdgcn_readfirstlane(len))) {
+      h = blk % H;
+      const int t = blk / H;
+      qb = t % n_qblk;
+      int k = t / n_qblk;
+      uint64_t m = ~0ull >> (64 - rank_b);
+      for (int bit = 31 - __builtin_clz(S); bit >= 0; --bit) {
+        const uint64_t has = m & __ballot(len >> bit & 1);
+        const int n = __builtin_popcountll(has);
+        const bool among = k < n;
+        m = among ? has : m & ~has;
+        k -= among ? 0 : n;
+      }
+      const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+      b = __builtin_ctzll(m & __ballot(at == k));
+    }
+    kvl = __builtin_amdgcn_readlane(len, b);
+  }
   const int d = H * HD;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, li = lane & 31;
-  int kvl = kv_len ? kv_len[b] : S;
-  kvl = kvl < 1 ? 1 : (kvl > S ? S : kvl);
+  if (kvl < 0) {
+    kvl = kv_len ? kv_len[b] : S;
+    kvl = kvl < 1 ? 1 : (kvl > S ? S : kvl);
+  }
   const int64_t row0 = seq_start ? (int64_t)seq_start[b] : (int64_t)b * S;
   const int lim = seq_start ? kvl : S;
   if (qb * BQ >= lim) return;
@@ -433,9 +451,16 @@ hipError_t attention(const AttnArgs &a, hipStream_t s) {
   const int force_logits = a.scale > 0.0f ? 0 : 1;  // raw-score max needs scale > 0
   // Sequences of uneven length without a launch order: the kernel ranks up to
   // 64 of them itself (one per lane), so that the long ones' blocks start first
-  // and no CU is left with several of them at the end: 17 sequences of up to 433
-  // rows, 12 heads of 64, 21.6 -> 18.5 us. (The packed passes give the order.)
-  const int rank_b = !a.order && a.kv_len && a.B > 1 && a.B <= 64 ? (int)a.B : 0;
+  // and no CU is left with several of them at the end. (The packed passes give
+  // the order.) In index order / ranked, lengths U[S/16, S], 12 heads of 64:
+  // 16 x 512 21.4 / 16.8 us, 32 x 512 35.8 / 30.4, 20 x 197 10.3 / 9.4,
+  // 16 x 2048 153 / 139; 64 x 128 of heads of 32 9.75 / 9.62. A launch whose
+  // blocks each have a CU gains nothing by it (8 x 256: 8.7 / 9.3, 2 x 512:
+  // 10.7 / 11.4), nor do shorter sequences (64 x 33: 4.5 / 5.3). Equal lengths
+  // keep the index order (32 x 512 44.8 / 45.3, 64 x 128 10.2 / 10.3).
+  const int rank_b =
+      !a.order && a.kv_len && a.B > 1 && a.B <= 64 && a.S >= 128 && blocks > cu_count() ? (int)a.B
+                                                                                      : 0;
   // head_dim 64: 32-key tiles, a 4-slot ring, four blocks per CU; head_dim 32:
   // 64-key tiles, 3 slots, three blocks per CU.
   if (a.hd == 64)

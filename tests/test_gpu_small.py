@@ -172,17 +172,24 @@ def test_small_gated_ffn(ctx, name, B, S):
         enc.close()
 
 
-@pytest.mark.parametrize("B,S,hd,lens", [
-    (2, 70, 64, [1, 70]),
-    (5, 200, 32, [200, 200, 3, 64, 129]),   # ties
-    (64, 40, 64, None),                     # the most sequences a wave ranks
-    (65, 40, 64, None),                     # one more: index order
+@pytest.mark.parametrize("B,S,hd,lens,H", [
+    (2, 70, 64, [1, 70], 2),
+    (5, 200, 32, [200, 200, 3, 64, 129], 2),   # ties
+    (64, 40, 64, None, 2),
+    (65, 40, 64, None, 2),
+    # ranked: more blocks than CUs, S of 128 or more
+    (2, 4200, 64, [1, 4200], 4),
+    (5, 1100, 32, [1100, 1100, 3, 64, 1099], 6),   # ties
+    (33, 128, 32, None, 9),                     # one query block
+    (64, 200, 64, None, 3),                     # the most sequences a wave ranks
+    (64, 200, 32, [200] * 64, 3),               # of one length: index order
+    (7, 257, 64, [0, 300, 257, 256, -5, 1, 128], 16),  # out of 1 .. S: clamped
+    (65, 200, 64, None, 3),                     # one more: index order
 ])
-def test_attention_ranks_uneven_sequences(ctx, B, S, hd, lens):
+def test_attention_ranks_uneven_sequences(ctx, B, S, hd, lens, H):
     """Attention over sequences of uneven length without a launch order: every
     sequence is computed once, bit for bit as when it is alone."""
-    print("case", B, S, hd, lens, flush=True)
-    H = 2
+    print("case", B, S, hd, lens, H, flush=True)
     d = H * hd
     rng = np.random.default_rng(B)
     lens = np.array(lens if lens else rng.integers(1, S + 1, B), np.int32)
