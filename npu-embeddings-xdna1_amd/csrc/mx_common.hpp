@@ -104,6 +104,15 @@ __device__ __forceinline__ float row_ror(float v) {
       __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + ROR, 0xF, 0xF, true));
 }
 
+// The last four steps: within each row of 16 lanes.
+template <class Op>
+__device__ __forceinline__ float row_butterfly(float v, Op op) {
+  v = op(v, row_ror<8>(v));
+  v = op(v, row_ror<4>(v));
+  v = op(v, row_ror<2>(v));
+  return op(v, row_ror<1>(v));
+}
+
 template <class Op>
 __device__ __forceinline__ float wave_butterfly(float v, Op op) {
   const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
@@ -111,20 +120,19 @@ __device__ __forceinline__ float wave_butterfly(float v, Op op) {
   v = op(__uint_as_float(h[0]), __uint_as_float(h[1]));
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
                                                   false);
-  v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  v = op(v, row_ror<8>(v));
-  v = op(v, row_ror<4>(v));
-  v = op(v, row_ror<2>(v));
-  return op(v, row_ror<1>(v));
+  return row_butterfly(op(__uint_as_float(r[0]), __uint_as_float(r[1])), op);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-  return wave_butterfly(v, [](float a, float b) { return a + b; });
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-  return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
-}
+struct AddOp {
+  __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+struct MaxOp {
+  __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+__device__ __forceinline__ float wave_sum(float v) { return wave_butterfly(v, AddOp()); }
+__device__ __forceinline__ float wave_max(float v) { return wave_butterfly(v, MaxOp()); }
+__device__ __forceinline__ float row_sum(float v) { return row_butterfly(v, AddOp()); }
+__device__ __forceinline__ float row_max(float v) { return row_butterfly(v, MaxOp()); }
 
 // gelu8 with the lane semantics of the reference's AVX2 branch
 // (bert_encoder.cpp:547-570): u = min(|v|, 4), degree-8 Horner by FMA, plus
