@@ -124,26 +124,29 @@ __global__ __launch_bounds__(256) void layernorm_quant_k(
       ia[i] = *(const float4 *)(ias + c);
     }
   }
-  // Every load of x, then every load of y, then the sums: a load behind the
-  // branch of the one before it would wait for its sum.
+  // Every load, then the sums: a load behind the branch of the one before it
+  // would wait for its sum. x and y in turn: with all of x first, 16,384 rows of
+  // 2048 took 93 us for 90.
   const int64_t at = row * cols + lane * 4;
   float4 v[NQ];
-#pragma unroll
-  for (int i = 0; i < NQ; ++i)
-    v[i] = i * 256 + lane * 4 < cols ? load4<ST>(x, false, at + i * 256)
+  auto ld = [&](const void *p, bool bf, int i) {
+    return i * 256 + lane * 4 < cols ? load4<ST>(p, bf, at + i * 256)
                                      : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  };
   if (y) {
     float4 w[NQ];
     if (y_bf) {
 #pragma unroll
-      for (int i = 0; i < NQ; ++i)
-        w[i] = i * 256 + lane * 4 < cols ? load4<ST>(y, true, at + i * 256)
-                                         : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      for (int i = 0; i < NQ; ++i) {
+        v[i] = ld(x, false, i);
+        w[i] = ld(y, true, i);
+      }
     } else {
 #pragma unroll
-      for (int i = 0; i < NQ; ++i)
-        w[i] = i * 256 + lane * 4 < cols ? load4<ST>(y, false, at + i * 256)
-                                         : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      for (int i = 0; i < NQ; ++i) {
+        v[i] = ld(x, false, i);
+        w[i] = ld(y, false, i);
+      }
     }
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
@@ -152,6 +155,9 @@ __global__ __launch_bounds__(256) void layernorm_quant_k(
       v[i].z += w[i].z;
       v[i].w += w[i].w;
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) v[i] = ld(x, false, i);
   }
   float s = 0.0f;
 #pragma unroll
