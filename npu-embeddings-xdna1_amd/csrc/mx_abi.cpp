@@ -248,7 +248,7 @@ int take_data_error(mx_stream *s, int *flags) {
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
   if (e != hipSuccess) return hip_fail(e, "reading the refusal flag");
   *flags = h[0];
-  s->saw_rows(h[1], s->plan_bound);
+  s->saw_rows(h[1], s->plan_B, s->plan_S);
   if (h[0]) {
     e = hipMemsetAsync(s->err_dev, 0, sizeof(int), s->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
@@ -342,8 +342,8 @@ int mx_stream_create(mx_ctx *ctx, mx_stream **out) {
     return hip_fail(e, "stream refusal flag");
   }
   // Only a hint rides on it: without pinned memory the stream goes on.
-  if (hipHostMalloc((void **)&s->note, sizeof(uint64_t), hipHostMallocDefault) == hipSuccess) {
-    *s->note = 0;
+  if (hipHostMalloc((void **)&s->note, 2 * sizeof(uint64_t), hipHostMallocDefault) == hipSuccess) {
+    s->note[0] = s->note[1] = 0;
   } else {
     s->note = nullptr;
     (void)hipGetLastError();

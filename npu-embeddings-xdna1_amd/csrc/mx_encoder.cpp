@@ -124,7 +124,7 @@ struct mx_encoder {
   // A packed pass whose row total stays on the device (no host wait in the
   // middle of the call): the launches over live_bound rows (the B * S the
   // workspace holds) take live -- the total's device address, and as the GEMM
-  // tile hint the stream's last total read with its refusal flag.
+  // tile hint the rows that the stream expects (mx_stream::expected_rows).
   mx::Live live;
   int64_t live_bound = 0;
   // timing
@@ -1349,8 +1349,11 @@ int pass_plan(mx_encoder *enc, Pass &p) {
   // the refusal flag at the end of the call: the next pass's tile hint.
   if (e == hipSuccess)
     e = mxk::pack_plan(p.w.kv_len, p.B, p.w.seq_start, p.w.seq_start + p.B + 1, p.s->stream,
-                       p.s->err_dev + 1, p.B > 1 ? p.s->note : nullptr, p.B * p.S);
-  if (e == hipSuccess) p.s->plan_bound = p.B > 1 ? p.B * p.S : 0;
+                       p.s->err_dev + 1, p.s->note ? p.s->note + (p.B == 1) : nullptr, p.B * p.S);
+  if (e == hipSuccess) {
+    p.s->plan_B = p.B;
+    p.s->plan_S = p.S;
+  }
   return e == hipSuccess ? MX_OK : hip_fail(e, "embed launch");
 }
 
@@ -1360,7 +1363,7 @@ int pass_plan(mx_encoder *enc, Pass &p) {
 // waits in the middle of the call. Three cases read it back instead: timing
 // (the whole plan, for the attention work), the static scratch (carve, which
 // takes the row-shaped buffers for exactly that many rows) and the first
-// packed pass on a stream (no earlier total to choose the GEMM tiles by).
+// packed batch on a stream (no earlier share to choose the GEMM tiles by).
 int pass_rows(mx_encoder *enc, Pass &p, Carver *carve) {
   Bracket br(enc, p.s->stream, CAT_OTHER);
   const int64_t B = p.B, S = p.S;
@@ -1382,15 +1385,15 @@ int pass_rows(mx_encoder *enc, Pass &p, Carver *carve) {
           enc->packed_sq += L * L;
         }
       }
-    } else if (carve || (B > 1 && p.s->last_rows <= 0)) {
-      // (also the first packed pass on a stream: no earlier total to pick the
-      // GEMM tiles by)
+    } else if (carve || (B > 1 && !p.s->seen_batch())) {
+      // (also the first packed batch on a stream: no earlier share to pick the
+      // GEMM tiles by; the first single sequence goes by its width)
       int32_t t = 0;
       e = hipMemcpyAsync(&t, p.w.seq_start + B, sizeof(int32_t), hipMemcpyDeviceToHost,
                          p.s->stream);
       if (e == hipSuccess) e = hipStreamSynchronize(p.s->stream);
       total = t;
-      if (e == hipSuccess) p.s->saw_rows(t, B > 1 ? B * S : 0);
+      if (e == hipSuccess) p.s->saw_rows(t, B, S);
     } else {
       enc->live = mx::Live{p.w.seq_start + B, p.s->expected_rows(B, S)};
       enc->live_bound = B * S;

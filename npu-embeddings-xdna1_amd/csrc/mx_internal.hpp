@@ -75,34 +75,40 @@ struct mx_stream {
   // Two device words: [0] the flags of kernels that refuse data, [1] the last
   // packed row total a pass planned on this stream.
   int *err_dev = nullptr;
-  // Word 1 as last read with the flags (host) and the B * S of the pass that
-  // wrote it: the share of a padded batch that is live, from which the next
-  // packed pass on this stream takes the row count its GEMM tiles are chosen
-  // for. (The bare count misjudges a pass of another size: batches of 64 x 512
-  // queued behind a query of three passages ran on the query's tiles, 6.1 ms a
-  // bge-base batch against 4.1.)
-  // A single sequence fills its own width and says nothing of a batch: it
-  // leaves the share as it was.
-  int last_rows = 0;
-  int64_t last_bound = 0;
-  int64_t plan_bound = 0;  // B * S of the last pass queued, 0 for one sequence
-  // The same pair as the last completed pass's plan wrote it (bound << 32 |
-  // rows, one 8-byte store into pinned host memory; 0 before the first), for
+  // The live share of the last passes on this stream, from which the next packed
+  // pass takes the row count its GEMM tiles are chosen for: word 1 as last read
+  // with the flags (host) and the B * S of the pass that wrote it. (The bare count
+  // misjudges a pass of another size: batches of 64 x 512 queued behind a query of
+  // three passages ran on the query's tiles, 6.1 ms a bge-base batch against 4.1.)
+  // [0] batches, [1] single sequences, which are padded to a fixed width or not
+  // at all whatever the batches' share is.
+  struct {
+    int rows = 0;
+    int64_t bound = 0;
+  } share[2];
+  int64_t plan_B = 0, plan_S = 0;  // the last pass queued
+  // The same pairs as the last completed pass's plan wrote them (bound << 32 |
+  // rows, one 8-byte store each into pinned host memory; 0 before the first), for
   // passes queued without a wait between them. Null: pinned memory refused.
   uint64_t *note = nullptr;
-  void saw_rows(int rows, int64_t bound) {
-    if (rows <= 0 || bound <= 0) return;
-    last_rows = rows;
-    last_bound = bound;
+  void saw_rows(int rows, int64_t B, int64_t S) {
+    if (rows <= 0 || B <= 0 || S <= 0) return;
+    share[B == 1].rows = rows;
+    share[B == 1].bound = B * S;
   }
+  bool seen_batch() const { return share[0].rows > 0; }
   int64_t expected_rows(int64_t B, int64_t S) {
     const int64_t bound = B * S;
+    auto &l = share[B == 1];
     if (note) {
-      const uint64_t v = __atomic_load_n(note, __ATOMIC_RELAXED);
-      saw_rows((int)(uint32_t)v, (int64_t)(v >> 32));
+      const uint64_t v = __atomic_load_n(note + (B == 1), __ATOMIC_RELAXED);
+      if ((uint32_t)v && v >> 32) {
+        l.rows = (int)(uint32_t)v;
+        l.bound = (int64_t)(v >> 32);
+      }
     }
-    if (B == 1 || last_bound <= 0) return bound;
-    const double r = (double)last_rows / (double)last_bound * (double)bound;
+    if (l.bound <= 0) return bound;
+    const double r = (double)l.rows / (double)l.bound * (double)bound;
     return r < 1.0 ? 1 : r < (double)bound ? (int64_t)r : bound;
   }
 };
@@ -175,7 +181,7 @@ int rope_checked(mx_stream *s, uint16_t *qkv, int64_t ld_qkv, int64_t B, int64_t
 int glu_checked(mx_stream *s, const void *up, int up_dtype, void *out, int out_dtype,
                 int64_t rows, int64_t f, int act, const Live &live = Live{});
 // Read and clear the stream's data-refusal flag (synchronises the stream);
-// word 1, the last packed row total, goes to s->last_rows.
+// word 1, the last packed row total, goes to s->share.
 int take_data_error(mx_stream *s, int *flags);
 // The static device scratch of mx_encoder_embed_static (mx_static.hip): its
 // address on each device is looked up once, by mx_create with that device

@@ -129,7 +129,7 @@ int collect(mx_embed_service *svc, Lane &l, Slot &sl, int64_t base, int64_t take
   const hipError_t e = hipEventSynchronize(sl.done);
   if (e != hipSuccess) return mx::hip_fail(e, "embed_service: waiting for a chunk");
   if (sl.flag[0]) return mx_sync(l.s);
-  if (take > 1) l.s->saw_rows(sl.flag[1], take * svc->seq);
+  l.s->saw_rows(sl.flag[1], take, svc->seq);
   const int64_t d = svc->hidden;
   std::memcpy(out + base * d, sl.out, static_cast<size_t>(take * d) * 4);
   return MX_OK;
