@@ -358,7 +358,7 @@ int cu_count() {
 
 
 const char *gemm_plan_name(int64_t M, int64_t N, int64_t K, bool c_bf16, bool residual,
-                           bool i8) {
+                           bool i8, bool gated) {
   static const float aligned_probe[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
   if (i8) {
     // The int8 kernels are the same tiles with slabs of 64 (or, deep, 128) int8.
@@ -368,6 +368,7 @@ const char *gemm_plan_name(int64_t M, int64_t N, int64_t K, bool c_bf16, bool re
     a.K = K;
     a.c_dtype = c_bf16 ? 1 : 0;
     a.residual = residual ? aligned_probe : nullptr;
+    a.epilogue = gated ? EPI_GLU_SILU : 0;
     const bool deep = gemm_i8_deep(a);
     switch (gemm_i8_tile(a)) {
       case 0:
@@ -390,6 +391,7 @@ const char *gemm_plan_name(int64_t M, int64_t N, int64_t K, bool c_bf16, bool re
   a.residual = residual ? aligned_probe : nullptr;
   a.C = (void *)aligned_probe;
   a.c_bf16 = c_bf16 ? 1 : 0;
+  a.epilogue = gated ? EPI_GLU_SILU : 0;
   switch (pick(a)) {
     case PATH_LDS_256x256_DEEP: return "lds_256x256x64_w64x128_ns2_persistent";
     case PATH_LDS_128x128_DEEP: return "lds_128x128x64_w64x64_ns2_persistent";

@@ -139,7 +139,8 @@ __host__ __device__ inline int balanced_grid(int ntiles, int grid) {
 }
 // The LDS-pipelined kernel addresses a lane's operand row within a tile as a
 // 32-bit byte offset from the tile origin: row r (< 256) of A at r * lda * esz
-// and of Wt at r * K * esz, plus at most 128 bytes of K. Both must stay below
+// and of Wt at r * K * esz, plus at most 240 bytes of K (the last chunk of a
+// 256-byte slab row). Both must stay below
 // 2^32, i.e. lda * esz and K * esz below 2^24.
 inline bool lds_offsets_fit(int64_t lda, int64_t K, int esz) {
   const int64_t lim = (int64_t)1 << 24;
@@ -210,9 +211,10 @@ hipError_t widen_i4_panel(const uint8_t *packed, int64_t K, int64_t N, int tile_
 // The plan the launcher would pick (for tests and reports): tile, slab depth
 // in K elements, wave tile and ring slots, e.g.
 // "lds_256x256x64_w64x128_ns2_persistent". gemm_config_name is the bf16
-// datapath's plan for an fp32 C without a residual.
+// datapath's plan for an fp32 C without a residual. gated: the fused gated FFN
+// (N = 2f; a bf16 C, no residual).
 const char *gemm_plan_name(int64_t M, int64_t N, int64_t K, bool c_bf16, bool residual,
-                           bool i8);
+                           bool i8, bool gated = false);
 const char *gemm_config_name(int64_t M, int64_t N, int64_t K);
 
 struct AttnArgs {

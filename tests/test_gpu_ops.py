@@ -403,10 +403,12 @@ GEMM_PATHS = [
     (16384, 768, 768, mxenc.MX_EPI_NONE, np.float32, True, "lds_256x192"),      # x += proj
     (16000, 768, 1532, mxenc.MX_EPI_GELU_ERF, np.float32, True, "lds_256x192"),  # ragged M, N
     (4096, 384, 1536, mxenc.MX_EPI_GELU_POLY, np.uint16, False, "lds_128x256"),  # MiniLM FFN-up
-    (1000, 1280, 3840, mxenc.MX_EPI_GELU_ERF, np.float32, True, "lds_128x128"),  # ragged M
+    (1000, 1280, 3840, mxenc.MX_EPI_GELU_ERF, np.float32, True,
+     "lds_128x128x64_w64x32_ns4_mfma16"),  # ragged M
     # bf16 C rows of 1004 are not 16-byte multiples: the register-staged kernel
     (777, 512, 1004, mxenc.MX_EPI_GELU_ERF, np.uint16, False, "staged_"),      # ragged M, N
-    (777, 512, 1000, mxenc.MX_EPI_GELU_ERF, np.uint16, False, "lds_128x128"),   # ragged M, N
+    (777, 512, 1000, mxenc.MX_EPI_GELU_ERF, np.uint16, False,
+     "lds_128x128x64_w64x32_ns4_mfma16"),   # ragged M, N
     # the 256 x 256 tile on 128-byte slabs (bf16 C, no residual, K % 64 == 0)
     (17455, 768, 2304, mxenc.MX_EPI_NONE, np.uint16, False, "lds_256x256x64"),  # packed QKV
     (17455, 3072, 768, mxenc.MX_EPI_NONE, np.uint16, False, "lds_256x256x64"),  # FFN-down
