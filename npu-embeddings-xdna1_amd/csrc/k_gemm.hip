@@ -218,17 +218,21 @@ bool lds_path_ok(const GemmArgs &a) {
 //        (+ n * res: an fp32 C with a residual),
 // `one` and `pair` the cost per K of one tile on a CU and of two: constants
 // fitted to products measured on an MI355X (weights rotating over eight copies),
-// but for the 128 x 256 row's cost per K, the best of four tried, and the 256 x
-// 256 row's cost per tile, raised from 3.28 for the sake of K below 512. Over
-// 700 further products (M 1 to 40,000, N 64 to 6144, K 128 to 5120; bf16, fp32 +
+// but for three: the 128 x 256 row's cost per K, the best of four tried; the 256
+// x 256 row's cost per tile, raised from 3.28 for the sake of K below 512; and the
+// 128 x 128 pairs' start, raised from 0.63, which leaves them and the 8-wave tile
+// level at one tile a CU and K = 384: repeated on the same operands the pairs are
+// faster (6000 x 384 x 384 7.0 us for 7.4), within a pass the 8-wave tile's three
+// slabs ahead are (MiniLM 32 x 128: 301 us a batch, 311 on the pairs). Over 700
+// further products (M 1 to 40,000, N 64 to 6144, K 128 to 5120; bf16, fp32 +
 // residual, gated) the choice takes 0.66 of the time of the choice by tile areas
-// over the 32 x 32 MFMA tiles alone, in the geometric mean, and the best tile of
-// each 0.66 too (1.009 between the two); the longest loses 3 % by it (38,303 x
-// 1000 x 1536, 111.9 -> 115.4 us). 700 x 1024 x 4096 takes 16.5 us for 42.2, 1500
-// x 768 x 768 7.9 for 11.1, 3000 x 1280 x 5120 with a residual 49.3 for 54.4, 300
-// x 768 x 128 4.55 for 4.88. The bounds on K keep a tile at least as deep as the
-// ring: a ring that held slabs of three tiles would hold two tiles' epilogue
-// vectors in one place. A 64-column tile over a ragged N is left out unmeasured.
+// over the 32 x 32 MFMA tiles alone, in the geometric mean, and 1.010 of the best
+// tile's; none of them takes over 1.2 % longer than by area. 700 x 1024 x 4096
+// takes 16.4 us for 42.2, 1500 x 768 x 768 7.9 for 11.1, 3000 x 1280 x 5120 with a
+// residual 49.7 for 54.7, 300 x 768 x 128 4.5 for 4.9. The bounds on K keep a tile
+// at least as deep as the ring: a ring that held slabs of three tiles would hold
+// two tiles' epilogue vectors in one place. A 64-column tile over a ragged N is
+// left out unmeasured.
 GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
   struct Cost {
     GemmPath path;
@@ -239,7 +243,7 @@ GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
       {PATH_LDS_256x256_DEEP, 256, 256, 3.27, .0198, .0396, 4.00, 3.84},
       {PATH_LDS_256x192, 256, 192, 1.73, .0183, .0366, 4.54, 2.54},
       {PATH_LDS_128x256, 128, 256, 0.00, .0150, .0300, 5.11, 1.73},
-      {PATH_LDS_128x128_DEEP, 128, 128, 0.63, .0103, .0135, 2.55, 2.64},
+      {PATH_LDS_128x128_DEEP, 128, 128, 0.85, .0103, .0135, 2.55, 2.64},
       {PATH_LDS16_128x128, 128, 128, 1.22, .0082, .0164, 2.94, 1.44},
       {PATH_LDS16_64x64_PAIR, 64, 64, 1.64, .0052, .0061, 0.86, 0.36},
       {PATH_LDS16_64x64, 64, 64, 2.16, .0036, .0072, 0.77, 1.14},

@@ -164,12 +164,15 @@ bool gemm_i8_deep(const GemmI8Args &a) {
 
 // The int8 product's tile (0 .. 3 as gemm_lds_tile, 4: 128 x 128 and 5: 64 x
 // 64 in 16 x 16 MFMAs): the least of us = start + n * (K * one + tile (+ wide: a
-// 4-byte C)) over n = ceil(tiles / CUs) rounds. Fitted to 190 products on an
-// MI355X (M 20 to 9000, K and N 384 to 5120; 6-13 % rms per tile), over which
-// the choice takes 0.77 of the time that the tile areas' choice took, and no
-// product longer: 4099 x 3072 x 768 with an fp32 C 24.3 -> 19.4 us, 300 x 3072
-// x 768 20.2 -> 8.3, 20 x 768 x 2304 8.1 -> 4.6. The bounds on K keep a tile as
-// deep as its ring, as for the bf16 forms (k_gemm.hip).
+// 4-byte C)) over n = ceil(tiles / CUs) rounds. The constants are fitted to
+// products measured on an MI355X. Over 191 further ones (M 1 to 40,000, N 64 to
+// 6144, K 256 to 5120; an fp32 C with or without a residual, or a bf16 C without)
+// the choice takes 0.77 of the time of the choice by tile areas over the 32 x 32
+// MFMA tiles alone, in the geometric mean, and none over 1 % longer: 4099 x 768 x
+// 3072 with an fp32 C 21.8 -> 17.7 us, 300 x 768 x 3072 19.5 -> 8.1, 20 x 2304 x
+// 768 with a bf16 C 7.4 -> 4.5. The raw product, bf16 + residual and the gated FFN
+// have the 32 x 32 tiles only. The bounds on K keep a tile as deep as its ring, as
+// for the bf16 forms (k_gemm.hip).
 int gemm_i8_tile(const GemmI8Args &a) {
   struct Cost {
     int bm, bn;
