@@ -203,7 +203,7 @@ def tiles_and_grid(plan, M, N):
 
 MANY = [
     # tile for, M, K, N, epilogue, bf16 C, residual, int8, kernel
-    (64, 9000, 384, 384, NONE, True, False, False, "lds_64x64x128_w32x32_ns3"),  # ring's depth
+    (64, 12000, 384, 384, NONE, True, False, False, "lds_64x64x128_w32x32_ns3"),  # ring's depth
     (1000, 6000, 896, 768, POLY, False, True, False, "lds_64x64x128_w32x32_ns3"),  # odd slabs
     (64, 9000, 256, 512, ERF, True, False, False, "lds_64x64x128_w32x32_ns2"),  # ring's depth
     (64, 9000, 640, 512, NONE, False, True, False, "lds_64x64x128_w32x32_ns2"),
