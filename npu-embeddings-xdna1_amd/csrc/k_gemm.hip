@@ -286,7 +286,8 @@ GemmPath pick_deep(int64_t M, int64_t N, int64_t K, bool res, bool glu) {
   }
   if (glu && best == PATH_LDS_128x128_DEEP) {
     // Few tiles of the gated FFN: 64 x 128 ones of 16 x 16 MFMAs while each has
-    // a CU (an even number of column blocks per wave, which 64 x 64 lacks).
+    // a CU (an even number of column blocks per wave, which 64 x 64 lacks). K 768,
+    // N 6144: 20 rows 8.2 us for 12.5, 320 rows (240 tiles) 11.8 for 13.9.
     if (K % 128 == 0 && K >= 384 && ((M + 63) / 64) * ((N + 127) / 128) <= cus)
       return PATH_LDS16_64x128_GLU;
     // The 64-byte form keeps three slabs in flight ahead, not one: a launch of
@@ -303,7 +304,8 @@ GemmPath pick(const GemmArgs &a) {
   const int64_t m = gemm_pick_rows(a.M, a.m_hint);
   const bool glu = a.epilogue >= EPI_GLU_SILU;
   if (deep_ok(a)) return pick_deep(m, a.N, a.K, a.residual != nullptr, glu);
-  // An fp32 C of few tiles (the ViT's patches): one small tile per CU.
+  // An fp32 C of few tiles (the ViT's patches): one small tile per CU, 300 x 768
+  // x 768 in 5.9 us for 11.7.
   if (!a.c_bf16 && !a.residual && a.epilogue == 0 && a.K % 128 == 0 && a.K >= 384 &&
       a.N % 64 == 0 &&
       ((a.M + 63) / 64) * (a.N / 64) <= cu_count())
@@ -345,7 +347,8 @@ int gemm_lds_tile(int64_t M, int64_t N) {
   return best;
 }
 
-// Resident blocks of the persistent kernel: one per CU of the current device.
+// The current device's CUs. A persistent launch has as many blocks, or twice as
+// many for the tiles of which two share a CU.
 int cu_count() {
   static int cached[64] = {0};
   int dev = 0;

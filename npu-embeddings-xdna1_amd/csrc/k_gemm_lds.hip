@@ -67,7 +67,7 @@ hipError_t gemm_lds_launch_t(const GemmArgs &a, int grid, hipStream_t s) {
 }
 
 // One tile configuration, every epilogue variant. `grid` = resident blocks
-// (one per CU).
+// (one per CU for these; the paired tiles below take twice as many).
 template <int BM, int BN, int WGM, int WGN, int NS>
 hipError_t gemm_lds_launch(const GemmArgs &a, int grid, hipStream_t s) {
   if (a.epilogue >= EPI_GLU_SILU) {
@@ -128,8 +128,8 @@ hipError_t gemm_lds_deep_launch(const GemmArgs &a, int grid, hipStream_t s) {
 // 64-byte form's four, half the barriers per K) for a bf16 C without a
 // residual or an fp32 C with one. 74-75 KB of LDS: two blocks share a CU, so
 // `grid` may be twice the CUs; the second block's MFMAs run under the first
-// one's barriers and epilogue (3940 x 1280 x 5120, fp32 C with a residual:
-// 94.8 us on the 64-byte form, 74.7 so; 6000 x 1280 x 5120, bf16 C: 110 -> 79).
+// one's barriers and epilogue (3940 rows, N 1280, K 5120, fp32 C with a
+// residual: 103.6 us on the 64-byte form, 71.8 so; 6000, bf16 C: 109 -> 79).
 hipError_t gemm_lds_128_deep_launch(const GemmArgs &a, int grid, hipStream_t s) {
   if (!a.c_bf16 && a.residual) {
     switch (a.epilogue) {

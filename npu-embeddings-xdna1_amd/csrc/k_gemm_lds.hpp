@@ -26,12 +26,13 @@
 // :874-900). With the bit set, the epilogue reads the accumulator through the
 // same rounding before anything else.
 //
-// Grid. One block per CU walks a list of BM x BN output tiles; its slabs
-// (RB = 64, 128 or 256 bytes of K per row: 32 or 64 bf16, 64 or 128 int8; 128-byte
-// rows make every load request a whole 128-byte line and halve the barriers
-// per K, and need two 64 KB slots for a 256 x 256 tile) form one sequence across tile
-// boundaries, so the ring keeps loading the next tile's first slabs while the
-// current tile drains: no per-tile prologue latency, no block relaunch.
+// Grid. One block per CU, or two where the launcher says so and both rings fit
+// its LDS, walks a list of BM x BN output tiles; its slabs (RB = 64, 128 or 256
+// bytes of K per row: 32, 64 or 128 bf16, 64, 128 or 256 int8; 128-byte rows make
+// every load request a whole 128-byte line and halve the barriers per K, and need
+// two 64 KB slots for a 256 x 256 tile) form one sequence across tile boundaries,
+// so the ring keeps loading the next tile's first slabs while the current tile
+// drains: no per-tile prologue latency, no block relaunch.
 // Workgroups go round-robin over the 8 XCDs, so the blocks of XCD x
 // (blockIdx % 8 == x) share the x-th eighth of the tiles (row-major over
 // (m, n)) and walk it together: they share A row-panels and W in that XCD's
@@ -55,7 +56,9 @@
 // they are on chip for the epilogue without a compiler-tracked load; the
 // waits do not count those loads, which only makes them stricter.
 //
-// Fragments. A slab is RB/32 k-steps of 32 bytes of K. Two register sets
+// Fragments (32 x 32 MFMAs; the 16 x 16 form below holds whole slabs instead, and
+// its barrier comes before a slab's MFMAs). A slab is RB/32 k-steps of 32 bytes of
+// K. Two register sets
 // alternate: each k-step's MFMAs run while the next k-step is read from LDS
 // into the other set (in the order the MFMAs consume it, one ds_read after
 // each of the first MFMAs, pinned by sched_group_barrier). The barrier sits
@@ -97,7 +100,7 @@
 // 49. The 16 x 16 form of 32 K adds the same products in the same order as two
 // 32 x 32 ones of 16 K: C's bits do not depend on the form. A 64 x 64 tile of
 // four such waves takes 0.15 us per 64 K against 0.63 for the 128 x 128 tile
-// that served small products before (100 x 4096 x 1024: 40.6 -> 15.5 us).
+// that served small products before (100 rows, K 4096, N 1024: 40.7 -> 15.3 us).
 //
 // Requirements (the launchers check them; bf16 shapes outside them go to
 // k_gemm.hip's kernel): K a multiple of the slab depth and at least NS slabs,
